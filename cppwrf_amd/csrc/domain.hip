@@ -272,7 +272,13 @@ struct Domain final : mi_domain {
 
   // SmallStep::run_stage (small_step.cpp:490-607); with prhophi, calc_p_rho_phi (small_step.cpp:609-617)
   // is fused into the finishing kernel.  In four parts, which a batch interleaves with its members' (ss_begin, then
-  // per substep advance_uv, after_uv, the column kernel, after_acoustic, then ss_end).
+  // per substep advance_uv, the column kernel and after_acoustic, then ss_end).
+  //
+  // No kernel between the stage's prologue and its end reads a halo point: the substep kernels reach their neighbour
+  // columns through the lateral boundary condition (a periodic side's column n is column 0, a mirrored or copied one
+  // its inner column).  So the reference's refreshes after the prologue, after advance_uv and after advance_mu_t and
+  // advance_w (small_step.cpp:517-522, 540-541, 572, 593) are left out: 21 launches of a dry step with 6 acoustic steps.
+  // The stage's last refreshes write every halo a later kernel reads.
   int stage_ns(int rk) const { return rk == 1 ? 1 : (rk == 2 ? n_sound_ / 2 : n_sound_); }
   double stage_dts(int rk) const { return rk == 1 ? grid.dt / 3.0 : grid.dt / n_sound_; }
   void small_steps(int rk, bool prhophi) {
@@ -281,7 +287,6 @@ struct Domain final : mi_domain {
     ss_begin(rk);
     for (int it = 1; it <= ns; ++it) {
       launch_uv(a, dts, stream());
-      after_uv();
       launch_acoustic(a, colcfg[kColAcoustic], dts, it, ns, stream());
       after_acoustic(rk, it);
     }
@@ -295,33 +300,10 @@ struct Domain final : mi_domain {
     launch_ss_prep(a, rk == 1, st);
     const double cof_h = 0.5 * dts * kG * (1.0 + prm.epssm);
     launch_ss_column(a, colcfg[kColSsColumn], cof_h * cof_h, dts, st);
-    // the halos of u'', v'', ph'', t_save, u_save, v_save, mu'', muts, p, al (small_step.cpp:517-522), in
-    // one batch after the two kernels: the column kernel reads its inputs in its own column only.  With
-    // specified boundaries no substep kernel reads them (as the substep refreshes below)
-    if (!spec)
-      halo({{f.u2, -1, -1}, {f.v2, -1, -1}, {f.ph2, -1, -1}, {f.t_save, -1, -1}, {f.u_save, -1, -1},
-            {f.v_save, -1, -1}, {f.mu2, -1, -1}, {f.muts, -1, -1}, {f.p, -1, -1}, {f.al, -1, -1}});
   }
-  // With specified boundaries the substep refreshes below are left out: no kernel of the substeps reads those halo
-  // points (the spec zone's faces and columns are advanced from their own values, the interior's stencils reach
-  // the spec zone only), and the stage's last refreshes write them before any reader.
-  bool needs_after_uv() const { return !spec; }
-  void after_uv() {
-    auto& f = a.f;
-    if (spec) {
-    } else if (!a.g.two_d) {
-      halo({{f.u2, -1, -1}, {f.v2, -1, -1}});  // small_step.cpp:540-541
-    } else {
-      halo({{f.u2, -1, -1}});
-    }
-  }
-  // after the substep's column kernel: the spec zone's columns, and the refreshes of mu'', mudf, muts and of ph'', p,
-  // al (small_step.cpp:572, 593)
+  // after the substep's column kernel: the spec zone's columns
   void after_acoustic(int rk, int it) {
-    auto& f = a.f;
     if (spec) launch_acoustic_ring(a, stage_dts(rk), it, stage_ns(rk), stream());
-    if (!spec)
-      halo({{f.mu2, -1, -1}, {f.mudf, -1, -1}, {f.muts, -1, -1}, {f.ph2, -1, -1}, {f.p, -1, -1}, {f.al, -1, -1}});
   }
   void ss_end(int rk, bool prhophi) {
     auto& f = a.f;
@@ -907,8 +889,6 @@ void build_domain(Domain& d, mi_ctx* ctx, const mi_grid& g, const mi_params& p, 
   add3(f.u_save, St::U, -1); add3(f.v_save, St::V, -1); add3(f.w_save, St::W, -1); add3(f.t_save, St::M, -1);
   add3(f.ph_save, St::W, -1); add3(f.ww1, St::W, -1); add3(f.c2a, St::M, -1); add3(f.pm1, St::M, -1);
   add3(f.ca, St::W, -1); add3(f.calpha, St::W, -1); add3(f.cgamma, St::W, -1);
-  add3(f.ky, St::W, -1);  // the scratch of the substep k-march
-  add3(f.kr, St::W, -1);
   add2(f.mu_save, St::M2, -1); add2(f.mudf, St::M2, -1); add2(f.muave, St::M2, -1);
   add2(f.mub, St::M2, MI_MUB);
   add2(f.msftx, St::M2, MI_MSFTX); add2(f.msfty, St::M2, MI_MSFTY);
@@ -1433,8 +1413,6 @@ void fused_capture(mi_domain* const* ms, int n, hipStream_t s0, const hipStream_
       hip_check(hipStreamWaitEvent(s0, join[q], 0), "hipStreamWaitEvent");
     }
   };
-  bool any_after_uv = false;
-  for (Domain* m : d) any_after_uv = any_after_uv || m->needs_after_uv();
   try {
     branch([](Domain& m) { m.step_begin(); });
     for (int rk = 1; rk <= 3; ++rk) {
@@ -1446,7 +1424,6 @@ void fused_capture(mi_domain* const* ms, int n, hipStream_t s0, const hipStream_
       });
       for (int it = 1; it <= ns; ++it) {
         launch_uv_batch(dev_args, tabs + size_t(rk - 1) * size_t(n + 1), n, info.blocks_uv[rk - 1], s0);
-        if (any_after_uv) branch([](Domain& m) { m.after_uv(); });
         launch_acoustic_batch(dev_args, tabs + size_t(rk + 2) * size_t(n + 1), n, info.blocks_ac[rk - 1], info.nzmax, it, ns,
                               s0);
         branch([rk, it](Domain& m) {

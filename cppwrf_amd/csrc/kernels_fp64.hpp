@@ -60,8 +60,6 @@ struct Fields {
   double *pd_dx, *pd_dxdt, *pd_dy, *pd_dydt, *pd_dz;
   // the advective forcings a column physics plugin asks for (WRF RTHFTEN, RQVFTEN); null when not wanted
   real *thf, *qvf;
-  // the substep k-march's scratch: the forward sweep's values and the explicit phi'' of the substep (FP64)
-  double *ky, *kr;
   // the diffusion's base state: theta's t_init (3-D), the 1-D profiles u_base, v_base, qv_base (nz values)
   BField t_init;
   double *u_base, *v_base, *qv_base;
@@ -180,9 +178,9 @@ constexpr int kNumColCfgs = 13;
 constexpr int kColCfgs[kNumColCfgs][2] = {{16, 16}, {16, 32}, {32, 16}, {8, 32}, {8, 64}, {4, 128}, {2, 256},
                                           {64, 4}, {64, 8}, {64, 16}, {32, 8}, {16, 64}, {4, 64}};
 constexpr int kColCfgTallest = 6;  // 2 x 256: the most levels per column (the substep kernel's nz limit)
-// one more shape of the substep kernel: one thread per column marching k (k_acoustic_march)
-constexpr int kColMarch = kNumColCfgs;
-constexpr int kNumColShapes = kColMarch + 1;
+// one more shape of the substep kernel: several levels per thread (k_acoustic_levels)
+constexpr int kColLevels = kNumColCfgs;
+constexpr int kNumColShapes = kColLevels + 1;
 constexpr const char* kColKernelNames[kNumColKernels] = {"large_prep", "ss_column", "acoustic", "finish"};
 bool col_cfg_fits(int kernel, int cfg, int nz);
 int col_cfg_default(int kernel, int nx, int ny, int nz);

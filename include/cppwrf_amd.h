@@ -418,7 +418,7 @@ int mi_domain_autotune(mi_domain* d, int trials);
 int mi_domain_get_tuning(const mi_domain* d, int* shapes, int n);
 /* sets the shapes explicitly (index 0..12 of the library's table of columns x threads per column: 16x16,
  * 16x32, 32x16, 8x32, 8x64, 4x128, 2x256, 64x4, 64x8, 64x16, 32x8, 16x64, 4x64; the substep kernel needs at
- * least nz+1 threads per column, or index 13: one thread per column marching k; MI_EINVAL if a shape does not
+ * least nz+1 threads per column, or index 13: several levels per thread; MI_EINVAL if a shape does not
  * fit nz) */
 int mi_domain_set_tuning(mi_domain* d, const int* shapes, int n);
 
