@@ -179,14 +179,27 @@ void launch3(const char* name, K kern, const Range& r, hipStream_t st, T... args
 }
 // A level-piece kernel over the points of r: a thread takes lv consecutive levels.  Long pieces share more between
 // levels; short ones keep enough wavefronts (about four per SIMD) on a small grid.
-int piece_levels(const Range& r, int by) {
-  const int64_t waves = int64_t(grid_of(r, by).x) * grid_of(r, by).y * by;  // per level
+int piece_levels(const Range& r, int by, int nsp = 1) {
+  const int64_t waves = int64_t(grid_of(r, by).x) * grid_of(r, by).y * by * nsp;  // per level
   const int64_t want = 4096;
   const int n = r.k1 - r.k0;
   int64_t lv = waves * n / want;
   lv = lv < 1 ? 1 : (lv > 16 ? 16 : lv);
   const int pieces = (n + int(lv) - 1) / int(lv);
   return (n + pieces - 1) / pieces;  // even pieces
+}
+// a scalar kernel over the points of r for each of nsp species (grid z = level pieces x species)
+template <class K, class... T>
+void launch_sc_pieces(const char* name, double arrays, K kern, Range r, int nsp, hipStream_t st, T... args) {
+  if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0 || nsp <= 0) return;
+  const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
+  const int lv = piece_levels(r, by, nsp);
+  dim3 gr = grid_of(r, by);
+  gr.z = unsigned((r.k1 - r.k0 + lv - 1) / lv) * unsigned(nsp);
+  const bool t = timing(name);
+  if (t) time_begin(st);
+  hipLaunchKernelGGL(kern, gr, dim3(kBx, by, 1), 0, st, r, lv, args...);
+  if (t) time_end(st, double(sizeof(real)) * arrays * double(r.i1 - r.i0) * double(r.j1 - r.j0) * double(r.k1 - r.k0));
 }
 template <class K, class... T>
 void launch_pieces(const char* name, double bytes, K kern, Range r, hipStream_t st, T... args) {
@@ -3492,14 +3505,229 @@ __device__ __forceinline__ acc m_full(const Lv& c, int k, double mub, double mu)
   return acc(c.c1h[k]) * (acc(mub) + acc(mu)) + acc(c.c2h[k]);
 }
 
-// rk_update_scalar (KUpdate, scalars.cpp:145-158): advect_scalar's tendency and the mass-weighted update,
-// every species of the list; the new values go to the species' second buffer
-template <bool OPEN, bool QVF>
-MI_POINT_KERNEL k_sc_update(Range r, Args a, Scalars s, SpList l, double dt_rk) {
-  MI_POINT_INDEX_SP(r)
+// One species over the levels ka <= k < kb of the wavefront's 64 columns of row j, marching up: the vertical stencil
+// slides through registers and a level's upper face is the next one's lower, the 2-D fields and the species' pointers
+// are read once, and a level's loads are issued together, none of them conditional.  MODE 0: rk_update_scalar; 1: the
+// limiter's scale; 2: its update (below).  Every expression is the per-level code's.  For rows whose y faces have the domain's
+// own order (sc_inner); columns next to a specified or open x side pick their order lane by lane.
+// Bounded by latency: the loads in flight per wavefront (54-103 VGPRs in FP32-bulk; FP64 also by the flux operators'
+// divisions).  425x300x50, six species, per launch against one level per thread: FP32-bulk update 519 -> 310 us, limiter
+// scale 753 -> 392, limited update 916 -> 443; FP64 888 -> 656, 1254 -> 835, 1626 -> 1091.
+template <int MODE>
+__device__ __forceinline__ void sc_levels(const Args& a, const real* q, const real* qo, const real* scl, const real* qtw,
+                                          real* out, int i, int j, int ka, int kb, acc dt) {
+  constexpr bool PD = MODE != 0;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j);
+  const bool two_d = g.two_d;
+  const acc hup = acc(a.q.hup), vup = acc(a.q.vup), zero = 0;
+  const ScFaces fl{a, q, qo, dt, PD};
+  unsigned eo = unsigned(kLpad + i);
+  asm("" : "+v"(eo));
+  const idx_t rj = j * sj - kLpad;
+  auto at = [&](const real* p, idx_t row) {
+    return reinterpret_cast<const real*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(real)));
+  };
+  const int ox0 = ord_face(i, nx, g.flx()), ox1 = ord_face(i + 1, nx, g.flx());
+  const bool xin = __all(ox0 == 5 && ox1 == 5);
+  const bool scell = fl.spec_cell(i, j), ecell = fl.edge_cell(i, j);
+  // column values
+  const double mub = f.mub[x2], mu1 = f.mu1[x2], mu2 = f.mu2[x2];
+  const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]), mxy = msftx * msfty;
+  const acc mx = msftx * acc(c.rdx), my = msftx * acc(c.rdy);
+  acc mt0 = 0, mtw = 0, mte = 0, mts_ = 0, mtn = 0, dx0 = 1, dx1 = 1, dy0 = 1, dy1 = 1, gx0 = 0, gx1 = 0, gy0 = 0, gy1 = 0;
+  if constexpr (PD) {
+    mt0 = acc(f.muts[x2]); mtw = acc(f.muts[x2 - 1]); mte = acc(f.muts[x2 + 1]);
+    mts_ = acc(f.muts[x2 - sj]); mtn = acc(f.muts[x2 + sj]);
+    dx0 = acc(f.pd_dx[x2]); dx1 = acc(f.pd_dx[x2 + 1]); dy0 = acc(f.pd_dy[x2]); dy1 = acc(f.pd_dy[x2 + sj]);
+    gx0 = acc(f.pd_dxdt[x2]); gx1 = acc(f.pd_dxdt[x2 + 1]); gy0 = acc(f.pd_dydt[x2]); gy1 = acc(f.pd_dydt[x2 + sj]);
+  }
+  auto flux_x = [&](int o, acc m3, acc m2, acc m1, acc q0, acc p1, acc p2, acc vel) -> acc {
+    if (o == 2) return acc(H) * vel * (q0 + m1);
+    if (o == 3) return vel * fl.f3(m2, m1, q0, p1, vel, hup);
+    return vel * fl.f5(m3, m2, m1, q0, p1, p2, vel);
+  };
+  auto face_z = [&](int kk, acc m2, acc m1, acc q0, acc p1, acc vel) -> acc {  // fz
+    if (kk == 0 || kk == nz) return zero;
+    if (kk == 1 || kk == nz - 1) return vel * (acc(c.fnm[kk]) * q0 + acc(c.fnp[kk]) * m1);
+    return vel * fl.f3(m2, m1, q0, p1, -vel, vup);
+  };
+  auto low_z = [&](int kk, acc om1, acc o0, acc vel) -> acc {  // fzl
+    if (kk == 0 || kk == nz) return zero;
+    const acc dz = acc(f.pd_dz[kk]), mu = acc(c.c1h[kk]) * mt0 + acc(c.c2h[kk]);
+    return mu * acc(f.pd_dz[nz + 1 + kk]) * flux_upwind<acc>(om1, o0, qdiv(qdiv(vel * dt, dz), mu));
+  };
+  auto lvl = [&](int k) { return rj + (k < 0 ? 0 : (k > nz ? nz : k)) * sk; };
+  // the window of levels ka - 2 .. ka + 1, and the lower face of ka
+  acc qm2 = at(q, lvl(ka - 2))[0], qm1 = at(q, lvl(ka - 1))[0], q0 = at(q, lvl(ka))[0], qp1 = at(q, lvl(ka + 1))[0];
+  acc om1 = 0, o0 = 0, s0 = 1, sm1 = 1, dhz0 = 0, loz0 = 0;
+  acc wz = at(f.ww_m, lvl(ka))[0];
+  acc fz0 = face_z(ka, qm2, qm1, q0, qp1, wz);
+  if constexpr (PD) {
+    om1 = at(qo, lvl(ka - 1))[0];
+    o0 = at(qo, lvl(ka))[0];
+    loz0 = low_z(ka, om1, o0, wz);
+    dhz0 = fz0 - loz0;
+  }
+  if constexpr (MODE == 2) {
+    s0 = at(scl, lvl(ka))[0];
+    sm1 = at(scl, lvl(ka - 1))[0];
+  }
+  for (int k = ka; k < kb; ++k) {
+    const idx_t r0 = rj + k * sk;
+    const real* qx = at(q, r0);
+    const acc xm3 = qx[-3], xm2 = qx[-2], xm1 = qx[-1], xp1 = qx[1], xp2 = qx[2], xp3 = qx[3];
+    const acc ym3 = at(q, r0 - 3 * sj)[0], ym2 = at(q, r0 - 2 * sj)[0], ym1 = at(q, r0 - sj)[0];
+    const acc yp1 = at(q, r0 + sj)[0], yp2 = at(q, r0 + 2 * sj)[0], yp3 = at(q, r0 + 3 * sj)[0];
+    const acc u0 = at(f.ru_m, r0)[0], u1 = at(f.ru_m, r0)[1], v0 = at(f.rv_m, r0)[0], v1 = at(f.rv_m, r0 + sj)[0];
+    const acc wzp = at(f.ww_m, r0 + sk)[0], qp2 = at(q, lvl(k + 2))[0];
+    acc oxm = 0, oxp = 0, oym = 0, oyp = 0, op1 = 0, old = 0, tq = 0, sxm = 1, sxp = 1, sym = 1, syp = 1, sp1 = 1;
+    if constexpr (PD) {
+      oxm = at(qo, r0)[-1]; oxp = at(qo, r0)[1]; oym = at(qo, r0 - sj)[0]; oyp = at(qo, r0 + sj)[0]; op1 = at(qo, lvl(k + 1))[0];
+    } else {
+      old = at(qo, r0)[0];
+      tq = at(qtw ? qtw : qo, r0)[0];
+    }
+    if constexpr (MODE == 2) {
+      sxm = at(scl, r0)[-1]; sxp = at(scl, r0)[1]; sym = at(scl, r0 - sj)[0]; syp = at(scl, r0 + sj)[0]; sp1 = at(scl, lvl(k + 1))[0];
+    }
+    const acc c1 = acc(c.c1h[k]), c2 = acc(c.c2h[k]), rdnw = acc(c.rdnw[k]);
+    acc fx0, fx1, fy0 = 0, fy1 = 0;
+    if (xin) {
+      fx0 = u0 * fl.f5(xm3, xm2, xm1, q0, xp1, xp2, u0);
+      fx1 = u1 * fl.f5(xm2, xm1, q0, xp1, xp2, xp3, u1);
+    } else {
+      fx0 = flux_x(ox0, xm3, xm2, xm1, q0, xp1, xp2, u0);
+      fx1 = flux_x(ox1, xm2, xm1, q0, xp1, xp2, xp3, u1);
+    }
+    if (!two_d) {
+      fy0 = v0 * fl.f5(ym3, ym2, ym1, q0, yp1, yp2, v0);
+      fy1 = v1 * fl.f5(ym2, ym1, q0, yp1, yp2, yp3, v1);
+    }
+    const acc fz1 = face_z(k + 1, qm1, q0, qp1, qp2, wzp);
+    if constexpr (MODE == 0) {
+      acc adv = 0;
+      if (!scell) {
+        adv = -mx * (fx1 - fx0);
+        if (!two_d) adv -= my * (fy1 - fy0);
+        adv = adv - rdnw * (fz1 - fz0);
+      }
+      acc tend = adv * msfty;
+      tend += qtw ? tq : zero;
+      const acc m_old = m_full(c, k, mub, mu1), m_new = m_full(c, k, mub, mu2);
+      row_st(out, r0, eo, qdiv(m_old * old + dt * tend, m_new));
+    } else {
+      // the low-order fluxes of the six faces and the high-minus-low ones (pd_faces)
+      const acc h0 = c1 * mt0 + c2;
+      auto low_x = [&](acc mu_w, acc mu_e, acc dx, acc gx, acc qw, acc qe, acc vel, bool deg) -> acc {
+        const acc mu = acc(H) * (mu_e + mu_w);
+        const acc cr = deg ? qdiv(qdiv(vel, mu) * dt, dx) : qdiv(qdiv(vel * dt, dx), mu);
+        return mu * gx * flux_upwind<acc>(qw, qe, cr);
+      };
+      const acc hw = c1 * mtw + c2, he = c1 * mte + c2;
+      const acc lox0 = low_x(hw, h0, dx0, gx0, oxm, o0, u0, g.flx() && i == 1), dhx0 = fx0 - lox0;
+      const acc lox1 = low_x(h0, he, dx1, gx1, o0, oxp, u1, g.flx() && i == 0), dhx1 = fx1 - lox1;
+      acc loy0 = 0, dhy0 = 0, loy1 = 0, dhy1 = 0;
+      if (!two_d) {
+        const acc hs = c1 * mts_ + c2, hn = c1 * mtn + c2;
+        loy0 = low_x(hs, h0, dy0, gy0, oym, o0, v0, false);
+        dhy0 = fy0 - loy0;
+        loy1 = low_x(h0, hn, dy1, gy1, o0, oyp, v1, false);
+        dhy1 = fy1 - loy1;
+      }
+      const acc loz1 = low_z(k + 1, o0, op1, wzp), dhz1 = fz1 - loz1;
+      if constexpr (MODE == 1) {
+        acc hlow = acc(c.rdx) * (lox1 - lox0);
+        if (!two_d) hlow += acc(c.rdy) * (loy1 - loy0);
+        const acc ph_low = ((c1 * acc(mub) + c2) + c1 * acc(mu1)) * o0 - dt * (mxy * hlow + msfty * rdnw * (loz1 - loz0));
+        acc hout = acc(c.rdx) * ((dhx1 > zero ? dhx1 : zero) - (dhx0 < zero ? dhx0 : zero));
+        if (!two_d) hout += acc(c.rdy) * ((dhy1 > zero ? dhy1 : zero) - (dhy0 < zero ? dhy0 : zero));
+        const acc outf = mxy * hout + msfty * rdnw * ((dhz1 < zero ? dhz1 : zero) - (dhz0 > zero ? dhz0 : zero));
+        const acc flux_out = dt * outf;
+        acc sc = 1;
+        if (flux_out > ph_low) {
+          sc = qdiv(ph_low, flux_out + acc(1e-20));
+          if (sc < zero) sc = 0;
+        }
+        row_st(out, r0, eo, ecell ? acc(1) : sc);  // WRF limits interior cells only
+      } else {
+        // the limited flux of a face: scaled by the scale of the cell it leaves
+        auto lim = [](acc d, acc s_minus, acc s_plus) { return d * (d > acc(0) ? s_minus : (d < acc(0) ? s_plus : acc(1))); };
+        const acc lx0 = lim(dhx0, sxm, s0), lx1 = lim(dhx1, s0, sxp);
+        // eta decreases upward: a positive w-level flux leaves the cell above it
+        const acc lz0 = k == 0 ? zero : lim(dhz0, s0, sm1);
+        const acc lz1 = k + 1 == nz ? zero : lim(dhz1, sp1, s0);
+        acc tend = -rdnw * (lz1 - lz0 + loz1 - loz0);
+        tend -= msftx * (acc(c.rdx) * (lx1 - lx0 + lox1 - lox0));
+        if (!two_d) {
+          const acc ly0 = lim(dhy0, sym, s0), ly1 = lim(dhy1, s0, syp);
+          tend -= msftx * (acc(c.rdy) * (ly1 - ly0 + loy1 - loy0));
+        }
+        const acc m_old = m_full(c, k, mub, mu1), m_new = m_full(c, k, mub, mu2);
+        // the spec zone: only the held tendency, folded into q_1 before
+        row_st(out, r0, eo, qdiv(scell ? m_old * o0 : m_old * o0 + dt * (tend * msfty), m_new));
+        sm1 = s0;
+        s0 = sp1;
+      }
+      dhz0 = dhz1;
+      loz0 = loz1;
+      om1 = o0;
+      o0 = op1;
+    }
+    fz0 = fz1;
+    qm2 = qm1;
+    qm1 = q0;
+    q0 = qp1;
+    qp1 = qp2;
+    wz = wzp;
+  }
+}
+// whether the y faces j and j + 1 have the domain's own order and, with open boundaries compiled in, no lane of the
+// wavefront is an open column: sc_levels' rows
+template <bool OPEN>
+__device__ __forceinline__ bool sc_inner(const ScFaces& fl, const Geo& g, int i, int j) {
+  const bool y = ord_face(j, g.ny, g.fly()) == 5 && ord_face(j + 1, g.ny, g.fly()) == 5;
+  return y && !(OPEN && (fl.open_row(j) || __any(fl.open_col(i))));
+}
+// a block of the scalar kernels: a level piece (level_piece) of one species, z = piece + pieces * species
+struct ScPiece {
+  int i, j, ka, kb, sq;
+  bool on;
+};
+__device__ __forceinline__ ScPiece sc_piece(const Range& r, int lv) {
+  const Blk b = point_block(1);
+  const int np = (r.k1 - r.k0 + lv - 1) / lv;
+  ScPiece p;
+  p.i = r.i0 + b.x * kBx + int(threadIdx.x);
+  p.j = r.j0 + b.y * int(blockDim.y) + __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+  p.sq = b.z / np;
+  p.ka = r.k0 + (b.z % np) * lv;
+  p.kb = p.ka + lv < r.k1 ? p.ka + lv : r.k1;
+  p.on = p.i < r.i1 && p.j < r.j1;
+  return p;
+}
+
+// rk_update_scalar (KUpdate, scalars.cpp:145-158): advect_scalar's tendency and the mass-weighted update,
+// every species of the list; the new values go to the species' second buffer
+template <bool OPEN, bool QVF>
+MI_POINT_KERNEL k_sc_update(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
+  const ScPiece pc = sc_piece(r, lv);
+  if (!pc.on) return;
+  const Geo& g = a.g;
+  const Fields& f = a.f;
+  const Lv& c = a.c;
+  const int i = pc.i, j = pc.j, sq_ = pc.sq;
+  {
+    const int n = l.sp[sq_];
+    if (!(QVF && f.qvf && n == 0) && sc_inner<OPEN>(ScFaces{a, s.q2[n], s.q1[n], acc(dt_rk), false}, g, i, j)) {
+      sc_levels<0>(a, s.q2[n], s.q1[n], nullptr, a.q.use_tendf ? s.qtw[n] : nullptr, s.qn[n], i, j, pc.ka, pc.kb, acc(dt_rk));
+      return;
+    }
+  }
+  for (int k = pc.ka; k < pc.kb; ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j), x0 = g.at(i, j, 0);
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc m_old = m_full(c, k, f.mub[x2], f.mu1[x2]), m_new = m_full(c, k, f.mub[x2], f.mu2[x2]);
@@ -3533,6 +3761,7 @@ MI_POINT_KERNEL k_sc_update(Range r, Args a, Scalars s, SpList l, double dt_rk) 
     }
     tend += acc((a.q.use_tendf ? s.qtw[n][x] : real(0)));
     put<kHMass>(s.qn[n], g, i, j, k * g.sk, qdiv(m_old * acc(s.q1[n][x]) + acc(dt_rk) * tend, m_new));
+  }
   }
 }
 
@@ -3578,11 +3807,21 @@ __device__ __forceinline__ PdFaces pd_faces(const ScFaces& fl, const Geo& g, int
 
 // advect_scalar_pd's limiter (KScalePD, scalars.cpp:220-248): the scale of each cell's outgoing
 // high-minus-low fluxes (its halo is refreshed next, as scalars.cpp:411)
-MI_POINT_KERNEL k_sc_pd_scale(Range r, Args a, Scalars s, SpList l, double dt_rk) {
-  MI_POINT_INDEX_SP(r)
+MI_POINT_KERNEL k_sc_pd_scale(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
+  const ScPiece pc = sc_piece(r, lv);
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int i = pc.i, j = pc.j, sq_ = pc.sq;
+  {
+    const int n = l.sp[sq_];
+    if (sc_inner<false>(ScFaces{a, s.q2[n], s.q1[n], acc(dt_rk), true}, g, i, j)) {
+      sc_levels<1>(a, s.q2[n], s.q1[n], nullptr, nullptr, s.scale[n], i, j, pc.ka, pc.kb, acc(dt_rk));
+      return;
+    }
+  }
+  for (int k = pc.ka; k < pc.kb; ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc mxy = msftx * msfty;
@@ -3592,7 +3831,7 @@ MI_POINT_KERNEL k_sc_pd_scale(Range r, Args a, Scalars s, SpList l, double dt_rk
     const ScFaces fl{a, s.q2[n], s.q1[n], dt, true};
     if (fl.edge_cell(i, j)) {  // WRF limits interior cells only
       put<kHMass>(s.scale[n], g, i, j, k * g.sk, 1.0);
-      return;
+      continue;
     }
     const PdFaces p = pd_faces(fl, g, i, j, k);
     acc hlow = acc(c.rdx) * (p.lox1 - p.lox0);
@@ -3610,16 +3849,27 @@ MI_POINT_KERNEL k_sc_pd_scale(Range r, Args a, Scalars s, SpList l, double dt_rk
     }
     put<kHMass>(s.scale[n], g, i, j, k * g.sk, sc);
   }
+  }
 }
 
 // advect_scalar_pd's limited divergence and rk_update_scalar (KUpdatePD, scalars.cpp:252-291)
 template <bool OPEN, bool QVF>
-MI_POINT_KERNEL k_sc_pd_update(Range r, Args a, Scalars s, SpList l, double dt_rk) {
-  MI_POINT_INDEX_SP(r)
+MI_POINT_KERNEL k_sc_pd_update(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
+  const ScPiece pc = sc_piece(r, lv);
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
   const int nz = g.nz;
+  const int i = pc.i, j = pc.j, sq_ = pc.sq;
+  {
+    const int n = l.sp[sq_];
+    if (!(QVF && f.qvf && n == 0) && sc_inner<OPEN>(ScFaces{a, s.q2[n], s.q1[n], acc(dt_rk), true}, g, i, j)) {
+      sc_levels<2>(a, s.q2[n], s.q1[n], s.scale[n], nullptr, s.qn[n], i, j, pc.ka, pc.kb, acc(dt_rk));
+      return;
+    }
+  }
+  for (int k = pc.ka; k < pc.kb; ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j), sj = g.sj, sk = g.sk;
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc m_old = m_full(c, k, f.mub[x2], f.mu1[x2]), m_new = m_full(c, k, f.mub[x2], f.mu2[x2]);
@@ -3631,7 +3881,7 @@ MI_POINT_KERNEL k_sc_pd_update(Range r, Args a, Scalars s, SpList l, double dt_r
     const bool ften = QVF && f.qvf && n == 0;
     if (fl.spec_cell(i, j) && !ften) {  // the spec zone: only the held tendency, folded into q_1 before
       put<kHMass>(s.qn[n], g, i, j, k * sk, qdiv(m_old * acc(s.q1[n][x]), m_new));
-      return;
+      continue;
     }
     const PdFaces p = pd_faces(fl, g, i, j, k);
     // the limited flux of a face: scaled by the scale of the cell it leaves
@@ -3652,7 +3902,7 @@ MI_POINT_KERNEL k_sc_pd_update(Range r, Args a, Scalars s, SpList l, double dt_r
       }
       f.qvf[x] = t * msfty;
       put<kHMass>(s.qn[n], g, i, j, k * sk, qdiv(m_old * acc(s.q1[n][x]), m_new));
-      return;
+      continue;
     }
     acc tend;
     if ((OPEN && fl.open_col(i)) || (OPEN && fl.open_row(j))) {  // open: open terms (with q_1), vertical, x (not outer columns), y
@@ -3673,6 +3923,7 @@ MI_POINT_KERNEL k_sc_pd_update(Range r, Args a, Scalars s, SpList l, double dt_r
     }
     if (ften) f.qvf[x] = tend * msfty;
     put<kHMass>(s.qn[n], g, i, j, k * sk, qdiv(m_old * acc(s.q1[n][x]) + dt * (tend * msfty), m_new));
+  }
   }
 }
 
@@ -4241,12 +4492,12 @@ void launch_scalars(const Args& a, const Scalars& s, const int* sp, int n, int s
   // the open-boundary terms and the RQVFTEN store compiled in only where used
   const bool op = g.ox() || g.oy(), qv = a.f.qvf != nullptr;
   switch (step) {
-    case 0: launch3s("sc_update", 3 + 4 * n, op ? (qv ? k_sc_update<true, true> : k_sc_update<true, false>)
+    case 0: launch_sc_pieces("sc_update", 3 + 4 * n, op ? (qv ? k_sc_update<true, true> : k_sc_update<true, false>)
                                                   : (qv ? k_sc_update<false, true> : k_sc_update<false, false>),
                      r, n, st, a, s, l, dt_rk); break;        // q_2 q_1 q_tendf -> q_new
     case 1: launch3s("sc_pd_pre", 3 * n, k_sc_pd_pre, r, n, st, a, s, l, dt_rk); break;            // q_1 q_tendf -> q_1
-    case 2: launch3s("sc_pd_scale", 3 + 3 * n, k_sc_pd_scale, r, n, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
-    default: launch3s("sc_pd_update", 3 + 4 * n, op ? (qv ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
+    case 2: launch_sc_pieces("sc_pd_scale", 3 + 3 * n, k_sc_pd_scale, r, n, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
+    default: launch_sc_pieces("sc_pd_update", 3 + 4 * n, op ? (qv ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
                                                         : (qv ? k_sc_pd_update<false, true> : k_sc_pd_update<false, false>),
                       r, n, st, a, s, l, dt_rk); break; // q_2 q_1 scale -> q_new
   }
