@@ -190,10 +190,10 @@ int piece_levels(const Range& r, int by, int nsp = 1) {
 }
 // a scalar kernel over the points of r for each of nsp species (grid z = level pieces x species)
 template <class K, class... T>
-void launch_sc_pieces(const char* name, double arrays, K kern, Range r, int nsp, hipStream_t st, T... args) {
+void launch_sc_pieces(const char* name, double arrays, bool one_level, K kern, Range r, int nsp, hipStream_t st, T... args) {
   if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0 || nsp <= 0) return;
   const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
-  const int lv = piece_levels(r, by, nsp);
+  const int lv = one_level ? 1 : piece_levels(r, by, nsp);
   dim3 gr = grid_of(r, by);
   gr.z = unsigned((r.k1 - r.k0 + lv - 1) / lv) * unsigned(nsp);
   const bool t = timing(name);
@@ -213,6 +213,16 @@ void launch_pieces(const char* name, double bytes, K kern, Range r, hipStream_t 
   if (t) time_begin(st);
   hipLaunchKernelGGL(kern, gr, dim3(kBx, by, 1), 0, st, r, lv, args...);
   if (t) time_end(st, bytes * double(r.i1 - r.i0) * double(r.j1 - r.j0) * double(r.k1 - r.k0));
+}
+// the same kernels one level per thread
+template <class K, class... T>
+void launch_level(const char* name, K kern, Range r, hipStream_t st, T... args) {
+  if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0) return;
+  const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
+  const bool t = timing(name);
+  if (t) time_begin(st);
+  hipLaunchKernelGGL(kern, grid_of(r, by), dim3(kBx, by, 1), 0, st, r, 1, args...);
+  if (t) time_end(st, point_bytes(name) * double(r.i1 - r.i0) * double(r.j1 - r.j0) * double(r.k1 - r.k0));
 }
 template <class K, class... T>
 void launch_cols(const char* name, K kern, int nx, int ny, int nz, hipStream_t st, T... args) {
@@ -505,6 +515,34 @@ MI_COLUMN_KERNEL k_large_prep(Args a) {
   }
 }
 
+// ----------------------------------------------------------------------------- level pieces
+// A wavefront's view of the fields: 64 consecutive points of one row (j and k are the same for all its lanes), so an
+// access is a scalar row address + the lane's 32-bit offset from the row's start (8 points west of i = 0).
+template <class T>
+__device__ __forceinline__ T row_ld(const T* p, idx_t row, unsigned eo) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ void row_st(T* p, idx_t row, unsigned eo, double v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(p + row) + eo * unsigned(sizeof(T))) = T(v);
+}
+
+// A block of the level-piece kernels: 64 points of four rows (a wavefront per row) x lv levels; the block grid is
+// x tiles, y tiles, level pieces, dealt to the XCDs in eighths, the pieces of a tile back to back (point_block)
+struct Piece {
+  int i, j, ka, kb;
+  bool on;
+};
+__device__ __forceinline__ Piece level_piece(const Range& r, int lv) {
+  const Blk b = point_block(1);
+  Piece p;
+  p.i = r.i0 + b.x * kBx + int(threadIdx.x);
+  p.j = r.j0 + b.y * int(blockDim.y) + __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+  p.ka = r.k0 + b.z * lv;
+  p.kb = p.ka + lv < r.k1 ? p.ka + lv : r.k1;
+  p.on = p.i < r.i1 && p.j < r.j1;
+  return p;
+}
 // ----------------------------------------------------------------------------- rk_tendency
 // KTendU (large_step.cpp:152-264): advect_u + horizontal pressure gradient + curvature, interior faces
 // MapC::vxgm (large_step.cpp:121-124): the map-factor curvature term at the mass point of index y (2-D y2)
@@ -565,12 +603,386 @@ __device__ __forceinline__ double open_y_scalar(const Geo& g, const T* q, const 
   return rdy * (vb * (Q(qo, ny - 1) - Q(qo, ny - 2)) + Q(q, ny - 1) * (RV(ny) - RV(ny - 1)));
 }
 
-template <bool OPEN>
-MI_POINT_KERNEL k_tend_u(Range r, Args a) {
-  MI_POINT_INDEX(r)
+// The large-step tendencies over the levels ka <= k < kb of the wavefront's 64 columns of row j, marching up: vertical
+// stencils and the pressure and mass-flux values two levels share slide through registers, the 2-D fields and what is
+// formed from them are read once, and a level's loads are issued together, none of them conditional.  The expressions are
+// the per-level kernels' below, operand for operand; the marches take the rows whose y fluxes have the domain's own
+// order and the wavefronts without an open edge, the per-level code the others.  Columns next to a specified or open x
+// side pick their x flux's order lane by lane.
+struct Row {  // the row's accessors: p[d] at (i + d) of the row that starts at index row
+  unsigned eo;
+  template <class T>
+  __device__ __forceinline__ const T* operator()(const T* p, idx_t row) const {
+    return reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
+  }
+};
+__device__ __forceinline__ Row row_of(int i) {
+  unsigned eo = unsigned(kLpad + i);
+  asm("" : "+v"(eo));
+  return Row{eo};
+}
+// KTendU (DIR 0) and KTendV (DIR 1): the same terms with the two directions exchanged
+template <int DIR>
+__device__ __forceinline__ void tend_uv_levels(const Args& a, int i, int j, int ka, int kb) {
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int nz = g.nz;
+  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j);
+  const Row at = row_of(i);
+  const idx_t rj = j * sj - kLpad, rs = rj - sj;
+  const bool spx = g.flx(), sx = g.spec(), two_d = g.two_d, moist = a.q.moist != 0, cor = a.q.cor != 0, mapped = a.q.mapped != 0;
+  const acc hup = acc(a.q.hup), vup = acc(a.q.vup);
+  const real* w = DIR == 0 ? f.u2 : f.v2;  // the advected wind
+  // the point across the face: i - 1 (u) or j - 1 (v)
+  const idx_t rb = DIR == 0 ? rj : rs;
+  constexpr int db = DIR == 0 ? -1 : 0;
+  const idx_t y2 = DIR == 0 ? x2 - 1 : x2 - sj;
+  const int o0 = DIR == 0 ? ord_mass(i, g.nx, spx) : ord_face(i, g.nx, spx);
+  const int o1 = DIR == 0 ? ord_mass(i + 1, g.nx, spx) : ord_face(i + 1, g.nx, spx);
+  const bool xin = __all(o0 == 5 && o1 == 5);
+  // column values
+  const double msfx = DIR == 0 ? f.msfux[x2] : f.msfvy[x2], msfy = DIR == 0 ? f.msfuy[x2] : f.msfvx[x2];
+  const double rd = DIR == 0 ? c.rdx : c.rdy, rm = msfx / msfy;
+  const double mf = DIR == 0 ? f.muu[x2] : f.muv[x2], mu0 = f.mu2[x2], mub = f.mu2[y2];
+  const double ax = -(msfx * c.rdx), ay = msfx * c.rdy, g1 = rm * H * rd, g2 = rm * rd;
+  const double f1 = rm * H * (f.fcor[x2] + f.fcor[y2]);
+  const double f2 = DIR == 0 ? H * (f.ecor[x2] + f.ecor[y2]) * H * (f.cosa[x2] + f.cosa[y2])
+                             : rm * H * (f.ecor[x2] + f.ecor[y2]) * H * (f.sina[x2] + f.sina[y2]);
+  const double vx0 = f.msfvx[x2 + sj] - f.msfvx[x2], uy0 = f.msfuy[x2 + 1] - f.msfuy[x2];
+  const double vxb = f.msfvx[y2 + sj] - f.msfvx[y2], uyb = f.msfuy[y2 + 1] - f.msfuy[y2];
+  const double tf = DIR == 0 ? msfy : f.msfvx_inv[x2];
+  real* out = DIR == 0 ? f.ru_tend : f.rv_tend;
+  const real* held = DIR == 0 ? f.ru_tendf : f.rv_tendf;
+  const real* cq = DIR == 0 ? f.cqu : f.cqv;
+  auto psum = [&](int m) { return at(f.p, rb + m * sk)[db] + at(f.p, rj + m * sk)[0]; };
+  auto face_x = [&](int o, int fi, real m3, real m2, real m1, real q0, real p1, real p2, real r0, real r1) -> acc {
+    // r0, r1: the mass flux at the point and across
+    if (o == 2) {
+      if constexpr (DIR == 0) {
+        if (fi <= 1) {
+          const double ub = (sx && q0 < 0.0) ? double(q0) : double(m1);
+          return acc(Q * (r0 + r1) * (q0 + ub));
+        }
+        const double ub = (sx && m1 > 0.0) ? double(m1) : double(q0);
+        return acc(Q * (r0 + r1) * (m1 + ub));
+      } else {
+        return acc(Q * (r0 + r1) * (q0 + m1));
+      }
+    }
+    const acc vel = acc(H * (r0 + r1));
+    if (o == 3) return acc(vel * flux3<acc>(m2, m1, q0, p1, vel, hup));
+    return acc(vel * flux5<acc>(m3, m2, m1, q0, p1, p2, vel, hup));
+  };
+  auto face_z = [&](int kk, real m2, real m1, real q0, real p1, real wb, real w0) -> acc {
+    if (kk == 0 || kk == nz) return acc(0.0);
+    const acc vel = acc(H * (wb + w0));
+    if (kk == 1 || kk == nz - 1) return acc(vel * (c.fnm[kk] * q0 + c.fnp[kk] * m1));
+    return acc(vel * flux3<acc>(m2, m1, q0, p1, -vel, vup));
+  };
+  auto lvl = [&](int k) { return rj + (k < 0 ? 0 : (k > nz ? nz : k)) * sk; };
+  // level ka's lower values
+  const idx_t ra = rj + ka * sk, rba = rb + ka * sk;
+  real qm2 = at(w, lvl(ka - 2))[0], qm1 = at(w, lvl(ka - 1))[0], q0 = at(w, ra)[0], qp1 = at(w, lvl(ka + 1))[0];
+  real p0 = at(f.p, ra)[0], pb_ = at(f.p, rba)[db], h0 = at(f.ph2, ra)[0], hb = at(f.ph2, rba)[db];
+  real rw0 = at(f.rw, ra)[0], rwb = at(f.rw, rba)[db];
+  const real wwa = at(f.ww, ra)[0], wwb = at(f.ww, rba)[db];
+  acc fz0 = face_z(ka, qm2, qm1, q0, qp1, wwb, wwa);
+  double dn;
+  if (ka == 0) dn = H * (c.cf1 * psum(0) + c.cf2 * psum(1) + c.cf3 * psum(2));
+  else dn = H * (c.fnm[ka] * (pb_ + p0) + c.fnp[ka] * psum(ka - 1));
+  const idx_t pbj = f.pb.si ? rj : 0, pbb = f.pb.si ? rb : 0;
+  const unsigned pbo = f.pb.si ? at.eo : 0u, pbw = f.pb.si ? at.eo + unsigned(db) : 0u;
+  for (int k = ka; k < kb; ++k) {
+    const idx_t r0 = rj + k * sk, r1 = rb + k * sk, rsk = rs + k * sk;
+    const real* qx = at(w, r0);
+    const real xm3 = qx[-3], xm2 = qx[-2], xm1 = qx[-1], xp1 = qx[1], xp2 = qx[2], xp3 = qx[3];
+    const real ym3 = at(w, r0 - 3 * sj)[0], ym2 = at(w, r0 - 2 * sj)[0], ym1 = at(w, r0 - sj)[0];
+    const real yp1 = at(w, r0 + sj)[0], yp2 = at(w, r0 + 2 * sj)[0], yp3 = at(w, r0 + 3 * sj)[0];
+    // mass fluxes: u needs ru at i - 1, i, i + 1 and rv at (i - 1, i) x (j, j + 1); v the same with the directions exchanged
+    real ra0, ra1, ra2, rc00, rc01, rc10, rc11;
+    if constexpr (DIR == 0) {
+      ra0 = at(f.ru, r0)[-1]; ra1 = at(f.ru, r0)[0]; ra2 = at(f.ru, r0)[1];
+      rc00 = at(f.rv, r0)[-1]; rc01 = at(f.rv, r0)[0]; rc10 = at(f.rv, r0 + sj)[-1]; rc11 = at(f.rv, r0 + sj)[0];
+    } else {
+      ra0 = at(f.rv, rsk)[0]; ra1 = at(f.rv, r0)[0]; ra2 = at(f.rv, r0 + sj)[0];
+      rc00 = at(f.ru, rsk)[0]; rc01 = at(f.ru, r0)[0]; rc10 = at(f.ru, rsk)[1]; rc11 = at(f.ru, r0)[1];
+    }
+    const real qp2 = at(w, lvl(k + 2))[0];
+    const real ww0p = at(f.ww, r0 + sk)[0], wwbp = at(f.ww, r1 + sk)[db];
+    const real p0p = at(f.p, r0 + sk)[0], pbp = at(f.p, r1 + sk)[db], h0p = at(f.ph2, r0 + sk)[0], hbp = at(f.ph2, r1 + sk)[db];
+    const real rw0p = at(f.rw, r0 + sk)[0], rwbp = at(f.rw, r1 + sk)[db];
+    const real at0 = at(f.alt, r0)[0], atb = at(f.alt, r1)[db], al0 = at(f.al, r0)[0], alb_ = at(f.al, r1)[db];
+    const double fp0 = at(f.php, r0)[0], fpb = at(f.php, r1)[db];
+    const unsigned bk = unsigned(k) * unsigned(f.pb.sk);
+    const double pbv = row_ld(f.pb.p, pbj, pbo + bk), pbvb = row_ld(f.pb.p, pbb, pbw + bk);
+    const real cqk = at(moist ? cq : f.alt, r0)[0], hk = at(a.q.use_tendf ? held : f.alt, r0)[0];
+    // the cross wind of the curvature term: v at (i - 1, i) x (j, j + 1) for u, u at (i, i + 1) x (j - 1, j) for v
+    const real* cw = DIR == 0 ? f.v2 : f.u2;
+    real cw00, cw01, cw10, cw11;
+    if constexpr (DIR == 0) {
+      cw00 = at(cw, r0)[-1]; cw01 = at(cw, r0)[0]; cw10 = at(cw, r0 + sj)[-1]; cw11 = at(cw, r0 + sj)[0];
+    } else {
+      cw00 = at(cw, rsk)[0]; cw01 = at(cw, r0)[0]; cw10 = at(cw, rsk)[1]; cw11 = at(cw, r0)[1];
+    }
+    const double c1 = c.c1h[k], c2 = c.c2h[k], rdnw = c.rdnw[k];
+    acc fx0, fx1, fy0 = 0, fy1 = 0;
+    if constexpr (DIR == 0) {
+      if (xin) {
+        const acc va = acc(H * (ra1 + ra0)), vb = acc(H * (ra2 + ra1));
+        fx0 = acc(va * flux5<acc>(xm3, xm2, xm1, q0, xp1, xp2, va, hup));
+        fx1 = acc(vb * flux5<acc>(xm2, xm1, q0, xp1, xp2, xp3, vb, hup));
+      } else {
+        fx0 = face_x(o0, i, xm3, xm2, xm1, q0, xp1, xp2, ra1, ra0);
+        fx1 = face_x(o1, i + 1, xm2, xm1, q0, xp1, xp2, xp3, ra2, ra1);
+      }
+      if (!two_d) {
+        const acc va = acc(H * (rc01 + rc00)), vb = acc(H * (rc11 + rc10));
+        fy0 = acc(va * flux5<acc>(ym3, ym2, ym1, q0, yp1, yp2, va, hup));
+        fy1 = acc(vb * flux5<acc>(ym2, ym1, q0, yp1, yp2, yp3, vb, hup));
+      }
+    } else {
+      if (xin) {
+        const acc va = acc(H * (rc01 + rc00)), vb = acc(H * (rc11 + rc10));
+        fx0 = acc(va * flux5<acc>(xm3, xm2, xm1, q0, xp1, xp2, va, hup));
+        fx1 = acc(vb * flux5<acc>(xm2, xm1, q0, xp1, xp2, xp3, vb, hup));
+      } else {
+        fx0 = face_x(o0, i, xm3, xm2, xm1, q0, xp1, xp2, rc01, rc00);
+        fx1 = face_x(o1, i + 1, xm2, xm1, q0, xp1, xp2, xp3, rc11, rc10);
+      }
+      const acc va = acc(H * (ra1 + ra0)), vb = acc(H * (ra2 + ra1));
+      fy0 = acc(va * flux5<acc>(ym3, ym2, ym1, q0, yp1, yp2, va, hup));
+      fy1 = acc(vb * flux5<acc>(ym2, ym1, q0, yp1, yp2, yp3, vb, hup));
+    }
+    const acc fz1 = face_z(k + 1, qm1, q0, qp1, qp2, wwbp, ww0p);
+    double up;  // dpn(k + 1)
+    if (k + 1 == nz) up = a.q.top_lid ? H * (c.cfn * psum(nz - 1) + c.cfn1 * psum(nz - 2)) : 0.0;
+    else up = H * (c.fnm[k + 1] * (pbp + p0p) + c.fnp[k + 1] * (pb_ + p0));
+    double t = ax * (fx1 - fx0);
+    if (!two_d) t -= ay * (fy1 - fy0);
+    if constexpr (DIR == 0) t -= rdnw * (fz1 - fz0);
+    else t -= rm * rdnw * (fz1 - fz0);
+    double dp = g1 * (c1 * mf + c2) * ((h0p - hbp + h0 - hb) + (at0 + atb) * (p0 - pb_) + (al0 + alb_) * (pbv - pbvb));
+    dp += g2 * (fp0 - fpb) * (rdnw * (up - dn) - H * (c1 * mub + c1 * mu0));
+    t -= (moist ? cqk : 1.0) * dp;
+    // vxgm at the point and across (kernels of large_step.cpp:121-124)
+    if constexpr (DIR == 0) {
+      const double rv4 = Q * (rc10 + rc11 + rc00 + rc01), rw4 = Q * (rwbp + rwb + rw0p + rw0);
+      if (cor) t = t + f1 * rv4 - f2 * rw4;
+      if (mapped) {
+        const double v0 = H * (q0 + xp1) * vx0 * c.rdy - H * (cw01 + cw11) * uy0 * c.rdx;
+        const double vb = H * (xm1 + q0) * vxb * c.rdy - H * (cw00 + cw10) * uyb * c.rdx;
+        t = t + H * (v0 + vb) * rv4 - q0 * kReradius * rw4;
+      } else {
+        t = t - q0 * kReradius * rw4;
+      }
+      if (a.q.use_tendf) t += hk / tf;  // rk_addtend_dry
+    } else {
+      const double ru4 = Q * (rc01 + rc11 + rc00 + rc10), rw4 = Q * (rwbp + rwb + rw0p + rw0);
+      if (cor) t = t - f1 * ru4 + f2 * rw4;
+      if (mapped) {
+        const double v0 = H * (cw01 + cw11) * vx0 * c.rdy - H * (q0 + yp1) * uy0 * c.rdx;
+        const double vb = H * (cw00 + cw10) * vxb * c.rdy - H * (ym1 + q0) * uyb * c.rdx;
+        t = t - H * (v0 + vb) * ru4 - rm * q0 * kReradius * rw4;
+      } else {
+        t = t - rm * q0 * kReradius * rw4;
+      }
+      if (a.q.use_tendf) t += hk * tf;  // rk_addtend_dry
+    }
+    row_st(out, r0, at.eo, t);
+    fz0 = fz1;
+    dn = up;
+    qm2 = qm1; qm1 = q0; q0 = qp1; qp1 = qp2;
+    p0 = p0p; pb_ = pbp; h0 = h0p; hb = hbp; rw0 = rw0p; rwb = rwbp;
+  }
+}
+// KTendT
+__device__ __forceinline__ void tend_t_levels(const Args& a, int i, int j, int ka, int kb) {
+  const Geo& g = a.g;
+  const Fields& f = a.f;
+  const Lv& c = a.c;
+  const int nz = g.nz;
+  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j);
+  const Row at = row_of(i);
+  const idx_t rj = j * sj - kLpad;
+  const real* q = f.t2;
+  const bool two_d = g.two_d, moist = a.q.moist != 0, held = a.q.use_tendf != 0;
+  const acc hup = acc(a.q.hup), vup = acc(a.q.vup);
+  const int o0 = ord_face(i, g.nx, g.flx()), o1 = ord_face(i + 1, g.nx, g.flx());
+  const bool xin = __all(o0 == 5 && o1 == 5);
+  const double msftx = f.msftx[x2], msfty = f.msfty[x2], mut = f.mut[x2];
+  const double ax = -(msftx * c.rdx), ay = msftx * c.rdy;
+  auto face_x = [&](int o, real m3, real m2, real m1, real q0, real p1, real p2, acc vel) -> acc {
+    if (o == 2) return acc(H * vel * (q0 + m1));
+    if (o == 3) return acc(vel * flux3<acc>(m2, m1, q0, p1, vel, hup));
+    return acc(vel * flux5<acc>(m3, m2, m1, q0, p1, p2, vel, hup));
+  };
+  auto face_z = [&](int kk, real m2, real m1, real q0, real p1, acc vel) -> acc {
+    if (kk == 0 || kk == nz) return acc(0.0);
+    if (kk == 1 || kk == nz - 1) return acc(vel * (c.fnm[kk] * q0 + c.fnp[kk] * m1));
+    return acc(vel * flux3<acc>(m2, m1, q0, p1, -vel, vup));
+  };
+  auto lvl = [&](int k) { return rj + (k < 0 ? 0 : (k > nz ? nz : k)) * sk; };
+  real qm2 = at(q, lvl(ka - 2))[0], qm1 = at(q, lvl(ka - 1))[0], q0 = at(q, lvl(ka))[0], qp1 = at(q, lvl(ka + 1))[0];
+  acc fz0 = face_z(ka, qm2, qm1, q0, qp1, acc(at(f.ww, lvl(ka))[0]));
+  for (int k = ka; k < kb; ++k) {
+    const idx_t r0 = rj + k * sk;
+    const real* qx = at(q, r0);
+    const real xm3 = qx[-3], xm2 = qx[-2], xm1 = qx[-1], xp1 = qx[1], xp2 = qx[2], xp3 = qx[3];
+    const real ym3 = at(q, r0 - 3 * sj)[0], ym2 = at(q, r0 - 2 * sj)[0], ym1 = at(q, r0 - sj)[0];
+    const real yp1 = at(q, r0 + sj)[0], yp2 = at(q, r0 + 2 * sj)[0], yp3 = at(q, r0 + 3 * sj)[0];
+    const acc u0 = at(f.ru, r0)[0], u1 = at(f.ru, r0)[1], v0 = at(f.rv, r0)[0], v1 = at(f.rv, r0 + sj)[0];
+    const acc wp = at(f.ww, r0 + sk)[0];
+    const real qp2 = at(q, lvl(k + 2))[0];
+    const real hk = at(held ? f.t_tendf : q, r0)[0], hd = at(moist ? f.hdia : q, r0)[0];
+    acc fx0, fx1, fy0 = 0, fy1 = 0;
+    if (xin) {
+      fx0 = acc(u0 * flux5<acc>(xm3, xm2, xm1, q0, xp1, xp2, u0, hup));
+      fx1 = acc(u1 * flux5<acc>(xm2, xm1, q0, xp1, xp2, xp3, u1, hup));
+    } else {
+      fx0 = face_x(o0, xm3, xm2, xm1, q0, xp1, xp2, u0);
+      fx1 = face_x(o1, xm2, xm1, q0, xp1, xp2, xp3, u1);
+    }
+    if (!two_d) {
+      fy0 = acc(v0 * flux5<acc>(ym3, ym2, ym1, q0, yp1, yp2, v0, hup));
+      fy1 = acc(v1 * flux5<acc>(ym2, ym1, q0, yp1, yp2, yp3, v1, hup));
+    }
+    const acc fz1 = face_z(k + 1, qm1, q0, qp1, qp2, wp);
+    double rr = ax * (fx1 - fx0);
+    if (!two_d) rr -= ay * (fy1 - fy0);
+    rr -= c.rdnw[k] * (fz1 - fz0);
+    if (held) rr += hk / msfty;  // rk_addtend_dry
+    // rk_addtend_dry's coupled heating (large_step.cpp:557), with moisture
+    if (moist) rr += (c.c1h[k] * mut + c.c2h[k]) * hd / msfty;
+    row_st(f.t_tend, r0, at.eo, rr);
+    fz0 = fz1;
+    qm2 = qm1; qm1 = q0; q0 = qp1; qp1 = qp2;
+  }
+}
+// KTendW, w levels 1..nz
+__device__ __forceinline__ void tend_w_levels(const Args& a, int i, int j, int ka, int kb) {
+  const Geo& g = a.g;
+  const Fields& f = a.f;
+  const Lv& c = a.c;
+  const int nz = g.nz;
+  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j);
+  const Row at = row_of(i);
+  const idx_t rj = j * sj - kLpad;
+  const real* q = f.w2;
+  const bool two_d = g.two_d, moist = a.q.moist != 0, held = a.q.use_tendf != 0, cor = a.q.cor != 0;
+  const acc hup = acc(a.q.hup), vup = acc(a.q.vup);
+  const int o0 = ord_face(i, g.nx, g.flx()), o1 = ord_face(i + 1, g.nx, g.flx());
+  const bool xin = __all(o0 == 5 && o1 == 5);
+  const double msftx = f.msftx[x2], msfty = f.msfty[x2], mut = f.mut[x2], mu = f.mu2[x2], mub = f.mub[x2];
+  const double ax = -(msftx * c.rdx), ay = msftx * c.rdy, rmsft = 1.0 / msfty, rmt = msftx / msfty;
+  const double ec = f.ecor[x2], co = f.cosa[x2], si = f.sina[x2];
+  auto face_x = [&](int o, real m3, real m2, real m1, real q0, real p1, real p2, acc vel) -> acc {
+    if (o == 2) return acc(H * vel * (q0 + m1));
+    if (o == 3) return acc(vel * flux3<acc>(m2, m1, q0, p1, vel, hup));
+    return acc(vel * flux5<acc>(m3, m2, m1, q0, p1, p2, vel, hup));
+  };
+  auto face_z = [&](int m, real m1, real w0, real w1, real p2, real ww0, real ww1) -> acc {  // at mass level m
+    if (m == 0 || m == nz - 1) return acc(0.25 * (ww1 + ww0) * (w1 + w0));
+    const acc vel = acc(H * (ww1 + ww0));
+    return acc(vel * flux3<acc>(m1, w0, w1, p2, -vel, vup));
+  };
+  auto lvl = [&](int k) { return rj + (k < 0 ? 0 : (k > nz ? nz : k)) * sk; };
+  // the level below ka
+  const idx_t rm = rj + (ka - 1) * sk;
+  real qm1 = at(q, rm)[0], q0 = at(q, lvl(ka))[0], qp1 = at(q, lvl(ka + 1))[0];
+  real wwm = at(f.ww, rm)[0], ww0 = at(f.ww, lvl(ka))[0];
+  real um0 = at(f.ru, rm)[0], um1 = at(f.ru, rm)[1], vm0 = at(f.rv, rm)[0], vm1 = at(f.rv, rm + sj)[0];
+  real am0 = at(f.u2, rm)[0], am1 = at(f.u2, rm)[1], bm0 = at(f.v2, rm)[0], bm1 = at(f.v2, rm + sj)[0];
+  real pm = at(f.p, rm)[0];
+  acc fz0 = face_z(ka - 1, at(q, lvl(ka - 2))[0], qm1, q0, qp1, wwm, ww0);
+  for (int k = ka; k < kb; ++k) {
+    const idx_t r0 = rj + k * sk;
+    const real* qx = at(q, r0);
+    const real xm3 = qx[-3], xm2 = qx[-2], xm1 = qx[-1], xp1 = qx[1], xp2 = qx[2], xp3 = qx[3];
+    const real ym3 = at(q, r0 - 3 * sj)[0], ym2 = at(q, r0 - 2 * sj)[0], ym1 = at(q, r0 - sj)[0];
+    const real yp1 = at(q, r0 + sj)[0], yp2 = at(q, r0 + 2 * sj)[0], yp3 = at(q, r0 + 3 * sj)[0];
+    const real u0 = at(f.ru, r0)[0], u1 = at(f.ru, r0)[1], v0 = at(f.rv, r0)[0], v1 = at(f.rv, r0 + sj)[0];
+    const real a0 = at(f.u2, r0)[0], a1 = at(f.u2, r0)[1], b0 = at(f.v2, r0)[0], b1 = at(f.v2, r0 + sj)[0];
+    const real wwp = at(f.ww, lvl(k + 1))[0], qp2 = at(q, lvl(k + 2))[0], p0 = at(f.p, r0)[0];
+    const real cqk = at(moist ? f.cqw : q, k < nz ? r0 : r0 - sk)[0], hk = at(held ? f.rw_tendf : q, r0)[0];
+    acc vx0, vx1, vy0, vy1;  // the mass fluxes at the w level
+    if (k < nz) {
+      vx0 = acc(c.fnm[k] * u0 + c.fnp[k] * um0);
+      vx1 = acc(c.fnm[k] * u1 + c.fnp[k] * um1);
+      vy0 = acc(c.fnm[k] * v0 + c.fnp[k] * vm0);
+      vy1 = acc(c.fnm[k] * v1 + c.fnp[k] * vm1);
+    } else {  // extrapolated at the lid
+      const idx_t r2 = r0 - 2 * sk;
+      const double fm = 2.0 - c.fnm[nz - 1], fp = c.fnp[nz - 1];
+      vx0 = acc(fm * um0 - fp * at(f.ru, r2)[0]);
+      vx1 = acc(fm * um1 - fp * at(f.ru, r2)[1]);
+      vy0 = acc(fm * vm0 - fp * at(f.rv, r2)[0]);
+      vy1 = acc(fm * vm1 - fp * at(f.rv, r2 + sj)[0]);
+    }
+    acc fx0, fx1;
+    if (xin) {
+      fx0 = acc(vx0 * flux5<acc>(xm3, xm2, xm1, q0, xp1, xp2, vx0, hup));
+      fx1 = acc(vx1 * flux5<acc>(xm2, xm1, q0, xp1, xp2, xp3, vx1, hup));
+    } else {
+      fx0 = face_x(o0, xm3, xm2, xm1, q0, xp1, xp2, vx0);
+      fx1 = face_x(o1, xm2, xm1, q0, xp1, xp2, xp3, vx1);
+    }
+    double t = ax * (fx1 - fx0);
+    if (!two_d) {
+      const acc fy0 = acc(vy0 * flux5<acc>(ym3, ym2, ym1, q0, yp1, yp2, vy0, hup));
+      const acc fy1 = acc(vy1 * flux5<acc>(ym2, ym1, q0, yp1, yp2, yp3, vy1, hup));
+      t -= ay * (fy1 - fy0);
+    }
+    const double cqw = moist ? cqk : 0.0, cq1 = 1.0 / (1.0 + cqw), cq2 = cqw * cq1;
+    acc fz1 = fz0;
+    if (k < nz) {
+      fz1 = face_z(k, qm1, q0, qp1, qp2, ww0, wwp);
+      t -= c.rdn[k] * (fz1 - fz0);
+      t += rmsft * kG * (cq1 * c.rdn[k] * (p0 - pm) - c.c1f[k] * mu - cq2 * (c.c1f[k] * mub + c.c2f[k]));
+      if (a.q.wd_dt != 0.0) {
+        const double muf = c.c1f[k] * mut + c.c2f[k];
+        double cfl = ww0 / muf * c.rdnw[k] * a.q.wd_dt;
+        cfl = cfl < 0.0 ? -cfl : cfl;
+        if (cfl > 1.0) t = t - (q0 < 0.0 ? -1.0 : 1.0) * 0.3 * (cfl - a.q.w_crit) * muf;
+      }
+      const double ruw = H * (c.fnm[k] * (u0 + u1) + c.fnp[k] * (um0 + um1));
+      const double rvw = H * (c.fnm[k] * (v0 + v1) + c.fnp[k] * (vm0 + vm1));
+      if (cor) t = t + ec * (co * ruw - rmt * si * rvw);
+      const double uw = H * (c.fnm[k] * (a0 + a1) + c.fnp[k] * (am0 + am1));
+      const double vw = H * (c.fnm[k] * (b0 + b1) + c.fnp[k] * (bm0 + bm1));
+      t = t + kReradius * (ruw * uw + rmt * rvw * vw);
+    } else {
+      t += 2.0 * c.rdn[nz - 1] * fz0;
+      t += rmsft * kG * (cq1 * 2.0 * c.rdnw[nz - 1] * (-pm) - c.c1f[nz] * mu - cq2 * (c.c1f[nz] * mub + c.c2f[nz]));
+    }
+    if (held) t += hk / msfty;  // rk_addtend_dry
+    row_st(f.rw_tend, r0, at.eo, t);
+    fz0 = fz1;
+    qm1 = q0; q0 = qp1; qp1 = qp2;
+    wwm = ww0; ww0 = wwp; pm = p0;
+    um0 = u0; um1 = u1; vm0 = v0; vm1 = v1; am0 = a0; am1 = a1; bm0 = b0; bm1 = b1;
+  }
+}
+// whether the marches take this row: its y fluxes in the domain's own order (ord_mass for v's)
+template <bool VROW>
+__device__ __forceinline__ bool tend_inner(const Geo& g, int j) {
+  return VROW ? ord_mass(j, g.ny, g.fly()) == 5 && ord_mass(j + 1, g.ny, g.fly()) == 5
+              : ord_face(j, g.ny, g.fly()) == 5 && ord_face(j + 1, g.ny, g.fly()) == 5;
+}
+
+template <bool OPEN>
+MI_POINT_KERNEL k_tend_u(Range r, int lv, Args a) {
+  const Piece pc = level_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  if (!pc.on) return;
+  const Geo& g = a.g;
+  const Fields& f = a.f;
+  const Lv& c = a.c;
+  const int i = pc.i, j = pc.j;
+  if (!OPEN && tend_inner<false>(g, j)) {
+    tend_uv_levels<0>(a, i, j, pc.ka, pc.kb);
+    return;
+  }
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const int nz = g.nz;
   const idx_t sj = g.sj, sk = g.sk;
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
@@ -631,7 +1043,7 @@ MI_POINT_KERNEL k_tend_u(Range r, Args a) {
     if (!(OPEN && g.oy())) t -= c.rdnw[k] * (fz(k + 1) - fz(k));
     if (a.q.use_tendf) t += f.ru_tendf[x] / msfuy;  // rk_addtend_dry
     f.ru_tend[x] = t;
-    return;
+    continue;
   }
   double t = -(msfux * c.rdx) * (fx(x + 1, i + 1) - fx(x, i));
   if (!g.two_d) {
@@ -676,15 +1088,23 @@ MI_POINT_KERNEL k_tend_u(Range r, Args a) {
     t = t - u[x] * kReradius * rw4;
   if (a.q.use_tendf) t += f.ru_tendf[x] / msfuy;  // rk_addtend_dry
   f.ru_tend[x] = t;
+  }
 }
 
 // KTendV (large_step.cpp:267-376)
 template <bool OPEN>
-MI_POINT_KERNEL k_tend_v(Range r, Args a) {
-  MI_POINT_INDEX(r)
+MI_POINT_KERNEL k_tend_v(Range r, int lv, Args a) {
+  const Piece pc = level_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int i = pc.i, j = pc.j;
+  if (!OPEN && tend_inner<true>(g, j)) {
+    tend_uv_levels<1>(a, i, j, pc.ka, pc.kb);
+    return;
+  }
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const int nz = g.nz;
   const idx_t sj = g.sj, sk = g.sk;
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
@@ -742,7 +1162,7 @@ MI_POINT_KERNEL k_tend_v(Range r, Args a) {
     }
     if (a.q.use_tendf) t += f.rv_tendf[x] * f.msfvx_inv[x2];  // rk_addtend_dry
     f.rv_tend[x] = t;
-    return;
+    continue;
   }
   const double rm = msfvy / msfvx;
   double t;
@@ -789,15 +1209,23 @@ MI_POINT_KERNEL k_tend_v(Range r, Args a) {
     t = t - rm * v[x] * kReradius * rw4;
   if (a.q.use_tendf) t += f.rv_tendf[x] * f.msfvx_inv[x2];  // rk_addtend_dry
   f.rv_tend[x] = t;
+  }
 }
 
 // KTendW (large_step.cpp:379-499), w levels 1..nz
 template <bool OPEN>
-MI_POINT_KERNEL k_tend_w(Range r, Args a) {
-  MI_POINT_INDEX(r)
+MI_POINT_KERNEL k_tend_w(Range r, int lv, Args a) {
+  const Piece pc = level_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int i = pc.i, j = pc.j;
+  if (!OPEN && tend_inner<false>(g, j)) {
+    tend_w_levels(a, i, j, pc.ka, pc.kb);
+    return;
+  }
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const int nz = g.nz;
   const idx_t sj = g.sj, sk = g.sk;
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
@@ -916,15 +1344,23 @@ MI_POINT_KERNEL k_tend_w(Range r, Args a) {
   }
   if (a.q.use_tendf) t += f.rw_tendf[x] / msfty;  // rk_addtend_dry
   f.rw_tend[x] = t;
+  }
 }
 
 // KTendT (large_step.cpp:502-565)
 template <bool OPEN, bool THF>
-MI_POINT_KERNEL k_tend_t(Range r, Args a) {
-  MI_POINT_INDEX(r)
+MI_POINT_KERNEL k_tend_t(Range r, int lv, Args a) {
+  const Piece pc = level_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int i = pc.i, j = pc.j;
+  if (!OPEN && !(THF && f.thf) && tend_inner<false>(g, j)) {
+    tend_t_levels(a, i, j, pc.ka, pc.kb);
+    return;
+  }
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const int nz = g.nz;
   const idx_t sj = g.sj, sk = g.sk;
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
@@ -982,6 +1418,7 @@ MI_POINT_KERNEL k_tend_t(Range r, Args a) {
   // rk_addtend_dry's coupled heating (large_step.cpp:557), with moisture
   if (a.q.moist) rr += (c.c1h[k] * f.mut[x2] + c.c2h[k]) * f.hdia[x] / f.msfty[x2];
   f.t_tend[x] = rr;
+  }
 }
 
 // KTendPh rhs_ph (large_step.cpp:570-668), w levels 1..nz, 6th-order horizontal gradient
@@ -1284,17 +1721,6 @@ MI_COLUMN_KERNEL k_ss_column(Args a, double cof, double dts) {
 }
 
 // ----------------------------------------------------------------------------- advance_uv
-// A wavefront's view of the fields: 64 consecutive points of one row (j and k are the same for all its lanes), so an
-// access is a scalar row address + the lane's 32-bit offset from the row's start (8 points west of i = 0).
-template <class T>
-__device__ __forceinline__ T row_ld(const T* p, idx_t row, unsigned eo) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
-}
-template <class T>
-__device__ __forceinline__ void row_st(T* p, idx_t row, unsigned eo, double v) {
-  *reinterpret_cast<T*>(reinterpret_cast<char*>(p + row) + eo * unsigned(sizeof(T))) = T(v);
-}
-
 // KUV (small_step.cpp:151-190) of the levels ka <= k < kb of point (i, j), marching up: the pressure sums and the
 // geopotential differences of a level are the next one's lower values, the 2-D fields are read once per column piece.
 // The west and south neighbours are addressed through the boundary condition (a periodic side's point -1 is point
@@ -1427,22 +1853,6 @@ __device__ __forceinline__ void uv_levels(const Args& a, int i, int j, int ka, i
     h0 = h0p; hw = hwp; hs = hsp;
     dnu = upu; dnv = upv;
   }
-}
-// A block of the level-piece kernels: 64 points of four rows (a wavefront per row) x lv levels; the block grid is
-// x tiles, y tiles, level pieces, dealt to the XCDs in eighths, the pieces of a tile back to back (point_block)
-struct Piece {
-  int i, j, ka, kb;
-  bool on;
-};
-__device__ __forceinline__ Piece level_piece(const Range& r, int lv) {
-  const Blk b = point_block(1);
-  Piece p;
-  p.i = r.i0 + b.x * kBx + int(threadIdx.x);
-  p.j = r.j0 + b.y * int(blockDim.y) + __builtin_amdgcn_readfirstlane(int(threadIdx.y));
-  p.ka = r.k0 + b.z * lv;
-  p.kb = p.ka + lv < r.k1 ? p.ka + lv : r.k1;
-  p.on = p.i < r.i1 && p.j < r.j1;
-  return p;
 }
 template <bool OPEN>
 MI_POINT_KERNEL k_uv(Range r, int lv, Args a, double dts) {
@@ -3361,25 +3771,41 @@ MI_POINT_KERNEL k_set_w_surface(Range r, Args a) {
 
 // ----------------------------------------------------------------------------- calc_cq
 // KCq (reference src/dyn/large_step.cpp:127-148): per species, the two neighbours, WRF's order
-MI_POINT_KERNEL k_cq(Range r, Args a, Scalars s) {
-  MI_POINT_INDEX(r)
+// A level piece per thread: the 3 N loads of a level are issued together (a loop over the species with its pointer
+// loaded each time waited 18 times per point: 425x300x50 with six species 132 us per launch), and the level below
+// slides through registers.
+template <int N>
+MI_POINT_KERNEL k_cq(Range r, int lv, Args a, Scalars s) {
+  const Piece pc = level_piece(r, lv);
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
-  const idx_t x = g.at(i, j, k);
-  if (j < g.ny) {
-    double t = 0;
-    for (int q = 0; q < s.n_moist; ++q) t = t + s.q2[q][x] + s.q2[q][x - 1];
-    f.cqu[x] = 1.0 / (1.0 + 0.5 * t);
-  }
-  if (i < g.nx && j < g.nyv) {
-    double t = 0;
-    for (int q = 0; q < s.n_moist; ++q) t = t + s.q2[q][x] + s.q2[q][x - g.sj];
-    f.cqv[x] = 1.0 / (1.0 + 0.5 * t);
-  }
-  if (i < g.nx && j < g.ny && k >= 1) {
-    double t = 0;
-    for (int q = 0; q < s.n_moist; ++q) t = t + s.q2[q][x] + s.q2[q][x - g.sk];
-    f.cqw[x] = 0.5 * t;
+  const int i = pc.i, j = pc.j;
+  const Row at = row_of(i);
+  const idx_t rj = j * g.sj - kLpad, sj = g.sj, sk = g.sk;
+  real below[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) below[q] = at(s.q2[q], rj + (pc.ka > 0 ? pc.ka - 1 : 0) * sk)[0];
+  for (int k = pc.ka; k < pc.kb; ++k) {
+    const idx_t r0 = rj + k * sk;
+    real q0[N], qw[N], qs[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      q0[q] = at(s.q2[q], r0)[0];
+      qw[q] = at(s.q2[q], r0)[-1];
+      qs[q] = at(s.q2[q], r0 - sj)[0];
+    }
+    double tu = 0, tv = 0, tw = 0;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      tu = tu + q0[q] + qw[q];
+      tv = tv + q0[q] + qs[q];
+      tw = tw + q0[q] + below[q];
+      below[q] = q0[q];
+    }
+    if (j < g.ny) row_st(f.cqu, r0, at.eo, 1.0 / (1.0 + 0.5 * tu));
+    if (i < g.nx && j < g.nyv) row_st(f.cqv, r0, at.eo, 1.0 / (1.0 + 0.5 * tv));
+    if (i < g.nx && j < g.ny && k >= 1) row_st(f.cqw, r0, at.eo, 0.5 * tw);
   }
 }
 
@@ -3520,7 +3946,7 @@ __device__ __forceinline__ void sc_levels(const Args& a, const real* q, const re
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int nx = g.nx, nz = g.nz;
   const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j);
   const bool two_d = g.two_d;
   const acc hup = acc(a.q.hup), vup = acc(a.q.vup), zero = 0;
@@ -3685,12 +4111,9 @@ __device__ __forceinline__ void sc_levels(const Args& a, const real* q, const re
     wz = wzp;
   }
 }
-// whether the y faces j and j + 1 have the domain's own order and, with open boundaries compiled in, no lane of the
-// wavefront is an open column: sc_levels' rows
-template <bool OPEN>
-__device__ __forceinline__ bool sc_inner(const ScFaces& fl, const Geo& g, int i, int j) {
-  const bool y = ord_face(j, g.ny, g.fly()) == 5 && ord_face(j + 1, g.ny, g.fly()) == 5;
-  return y && !(OPEN && (fl.open_row(j) || __any(fl.open_col(i))));
+// whether the y faces j and j + 1 have the domain's own order: sc_levels' rows
+__device__ __forceinline__ bool sc_inner(const Geo& g, int j) {
+  return ord_face(j, g.ny, g.fly()) == 5 && ord_face(j + 1, g.ny, g.fly()) == 5;
 }
 // a block of the scalar kernels: a level piece (level_piece) of one species, z = piece + pieces * species
 struct ScPiece {
@@ -3714,7 +4137,7 @@ __device__ __forceinline__ ScPiece sc_piece(const Range& r, int lv) {
 // every species of the list; the new values go to the species' second buffer
 template <bool OPEN, bool QVF>
 MI_POINT_KERNEL k_sc_update(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
-  const ScPiece pc = sc_piece(r, lv);
+  const ScPiece pc = sc_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
   if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
@@ -3722,12 +4145,12 @@ MI_POINT_KERNEL k_sc_update(Range r, int lv, Args a, Scalars s, SpList l, double
   const int i = pc.i, j = pc.j, sq_ = pc.sq;
   {
     const int n = l.sp[sq_];
-    if (!(QVF && f.qvf && n == 0) && sc_inner<OPEN>(ScFaces{a, s.q2[n], s.q1[n], acc(dt_rk), false}, g, i, j)) {
+    if (!OPEN && !(QVF && f.qvf && n == 0) && sc_inner(g, j)) {
       sc_levels<0>(a, s.q2[n], s.q1[n], nullptr, a.q.use_tendf ? s.qtw[n] : nullptr, s.qn[n], i, j, pc.ka, pc.kb, acc(dt_rk));
       return;
     }
   }
-  for (int k = pc.ka; k < pc.kb; ++k) {
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j), x0 = g.at(i, j, 0);
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc m_old = m_full(c, k, f.mub[x2], f.mu1[x2]), m_new = m_full(c, k, f.mub[x2], f.mu2[x2]);
@@ -3816,7 +4239,7 @@ MI_POINT_KERNEL k_sc_pd_scale(Range r, int lv, Args a, Scalars s, SpList l, doub
   const int i = pc.i, j = pc.j, sq_ = pc.sq;
   {
     const int n = l.sp[sq_];
-    if (sc_inner<false>(ScFaces{a, s.q2[n], s.q1[n], acc(dt_rk), true}, g, i, j)) {
+    if (sc_inner(g, j)) {
       sc_levels<1>(a, s.q2[n], s.q1[n], nullptr, nullptr, s.scale[n], i, j, pc.ka, pc.kb, acc(dt_rk));
       return;
     }
@@ -3855,7 +4278,7 @@ MI_POINT_KERNEL k_sc_pd_scale(Range r, int lv, Args a, Scalars s, SpList l, doub
 // advect_scalar_pd's limited divergence and rk_update_scalar (KUpdatePD, scalars.cpp:252-291)
 template <bool OPEN, bool QVF>
 MI_POINT_KERNEL k_sc_pd_update(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
-  const ScPiece pc = sc_piece(r, lv);
+  const ScPiece pc = sc_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
   if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
@@ -3864,12 +4287,12 @@ MI_POINT_KERNEL k_sc_pd_update(Range r, int lv, Args a, Scalars s, SpList l, dou
   const int i = pc.i, j = pc.j, sq_ = pc.sq;
   {
     const int n = l.sp[sq_];
-    if (!(QVF && f.qvf && n == 0) && sc_inner<OPEN>(ScFaces{a, s.q2[n], s.q1[n], acc(dt_rk), true}, g, i, j)) {
+    if (!OPEN && !(QVF && f.qvf && n == 0) && sc_inner(g, j)) {
       sc_levels<2>(a, s.q2[n], s.q1[n], s.scale[n], nullptr, s.qn[n], i, j, pc.ka, pc.kb, acc(dt_rk));
       return;
     }
   }
-  for (int k = pc.ka; k < pc.kb; ++k) {
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j), sj = g.sj, sk = g.sk;
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc m_old = m_full(c, k, f.mub[x2], f.mu1[x2]), m_new = m_full(c, k, f.mub[x2], f.mu2[x2]);
@@ -4276,13 +4699,19 @@ void launch_tendencies(const Args& a, hipStream_t st) {
   // open boundaries: the boundary faces are advanced too (large_step.cpp:804-806)
   // the open-boundary code and the RTHFTEN store compiled in only where used
   const bool op = g.ox() || g.oy();
-  launch3("tend_u", op ? k_tend_u<true> : k_tend_u<false>, Range{g.ox() ? 0 : ui0, g.ox() ? g.nx + 1 : g.nx, 0, g.ny, 0, g.nz}, st, a);
+  // Level marches; with open sides, whose edge columns take their own terms, a level per thread (97x75x35 FP64, where
+  // every wavefront holds an open column: the step 0.89 ms that way, 0.96 with the march's code around it)
+  auto go = [&](const char* name, auto kern, const Range& r) {
+    if (op) launch_level(name, kern, r, st, a);
+    else launch_pieces(name, point_bytes(name), kern, r, st, a);
+  };
+  go("tend_u", op ? k_tend_u<true> : k_tend_u<false>, Range{g.ox() ? 0 : ui0, g.ox() ? g.nx + 1 : g.nx, 0, g.ny, 0, g.nz});
   if (!g.two_d)
-    launch3("tend_v", op ? k_tend_v<true> : k_tend_v<false>, Range{0, g.nx, g.oy() ? 0 : vj0, g.oy() ? g.ny + 1 : g.ny, 0, g.nz}, st, a);
-  launch3("tend_w", op ? k_tend_w<true> : k_tend_w<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1}, st, a);
-  launch3("tend_t", op ? (a.f.thf ? k_tend_t<true, true> : k_tend_t<true, false>)
-                       : (a.f.thf ? k_tend_t<false, true> : k_tend_t<false, false>),
-          Range{0, g.nx, 0, g.ny, 0, g.nz}, st, a);
+    go("tend_v", op ? k_tend_v<true> : k_tend_v<false>, Range{0, g.nx, g.oy() ? 0 : vj0, g.oy() ? g.ny + 1 : g.ny, 0, g.nz});
+  go("tend_w", op ? k_tend_w<true> : k_tend_w<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1});
+  go("tend_t", op ? (a.f.thf ? k_tend_t<true, true> : k_tend_t<true, false>)
+                  : (a.f.thf ? k_tend_t<false, true> : k_tend_t<false, false>),
+     Range{0, g.nx, 0, g.ny, 0, g.nz});
   launch3("tend_ph", op ? k_tend_ph<true> : k_tend_ph<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1}, st, a);
 }
 
@@ -4471,7 +4900,19 @@ void launch_cfl_scratch(const Args& a, unsigned long long* sp, hipStream_t st) {
 void launch_cq(const Args& a, const Scalars& s, hipStream_t st) {
   const Geo& g = a.g;
   // the moist species -> cqu, cqv, cqw
-  launch3a("cq", s.n_moist + 3, k_cq, Range{0, g.nx + 1, 0, g.nyv, 0, g.nz}, st, a, s);
+  const Range r{0, g.nx + 1, 0, g.nyv, 0, g.nz};
+  const double b = double(sizeof(real)) * (s.n_moist + 3);
+  static_assert(MI_MAX_MOIST == 8, "one case per count");
+  switch (s.n_moist) {
+    case 1: launch_pieces("cq", b, k_cq<1>, r, st, a, s); break;
+    case 2: launch_pieces("cq", b, k_cq<2>, r, st, a, s); break;
+    case 3: launch_pieces("cq", b, k_cq<3>, r, st, a, s); break;
+    case 4: launch_pieces("cq", b, k_cq<4>, r, st, a, s); break;
+    case 5: launch_pieces("cq", b, k_cq<5>, r, st, a, s); break;
+    case 6: launch_pieces("cq", b, k_cq<6>, r, st, a, s); break;
+    case 7: launch_pieces("cq", b, k_cq<7>, r, st, a, s); break;
+    default: launch_pieces("cq", b, k_cq<8>, r, st, a, s); break;
+  }
 }
 // the kernels of the scalar transport of the species sp[0..n) (step: 0 rk_update_scalar; 1, 2, 3 the
 // positive-definite pre-update, limiter scale and update); algorithmic arrays: the mass fluxes ru_m, rv_m,
@@ -4492,12 +4933,12 @@ void launch_scalars(const Args& a, const Scalars& s, const int* sp, int n, int s
   // the open-boundary terms and the RQVFTEN store compiled in only where used
   const bool op = g.ox() || g.oy(), qv = a.f.qvf != nullptr;
   switch (step) {
-    case 0: launch_sc_pieces("sc_update", 3 + 4 * n, op ? (qv ? k_sc_update<true, true> : k_sc_update<true, false>)
+    case 0: launch_sc_pieces("sc_update", 3 + 4 * n, op, op ? (qv ? k_sc_update<true, true> : k_sc_update<true, false>)
                                                   : (qv ? k_sc_update<false, true> : k_sc_update<false, false>),
                      r, n, st, a, s, l, dt_rk); break;        // q_2 q_1 q_tendf -> q_new
     case 1: launch3s("sc_pd_pre", 3 * n, k_sc_pd_pre, r, n, st, a, s, l, dt_rk); break;            // q_1 q_tendf -> q_1
-    case 2: launch_sc_pieces("sc_pd_scale", 3 + 3 * n, k_sc_pd_scale, r, n, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
-    default: launch_sc_pieces("sc_pd_update", 3 + 4 * n, op ? (qv ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
+    case 2: launch_sc_pieces("sc_pd_scale", 3 + 3 * n, false, k_sc_pd_scale, r, n, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
+    default: launch_sc_pieces("sc_pd_update", 3 + 4 * n, op, op ? (qv ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
                                                         : (qv ? k_sc_pd_update<false, true> : k_sc_pd_update<false, false>),
                       r, n, st, a, s, l, dt_rk); break; // q_2 q_1 scale -> q_new
   }
