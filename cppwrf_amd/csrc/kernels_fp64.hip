@@ -1422,12 +1422,112 @@ MI_POINT_KERNEL k_tend_t(Range r, int lv, Args a) {
 }
 
 // KTendPh rhs_ph (large_step.cpp:570-668), w levels 1..nz, 6th-order horizontal gradient
-template <bool OPEN>
-MI_POINT_KERNEL k_tend_ph(Range r, Args a) {
-  MI_POINT_INDEX(r)
+__device__ __forceinline__ void tend_ph_levels(const Args& a, int i, int j, int ka, int kb) {
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
+  const int nz = g.nz;
+  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j);
+  const Row at = row_of(i);
+  const idx_t rj = j * sj - kLpad;
+  const real *ph = f.ph2, *u = f.u2, *v = f.v2;
+  const bool two_d = g.two_d, full = f.phb.si != 0, sp = g.spec();
+  // the x gradient's order of the column (y's is 6 in these rows): 0 on the outer two columns of a specified or the outer
+  // one of an open side, 2 on the next in
+  const bool fx = g.flx();
+  const int ox = !fx ? 6 : (i <= 0 || i >= g.nx - 1 ? 0 : (i == 1 || i == g.nx - 2 ? 2 : (i == 2 || i == g.nx - 3 ? 0 : 6)));
+  const bool xin = __all(ox == 6);
+  const double msfty = f.msfty[x2], mut = f.mut[x2], muu0 = f.muu[x2], muu1 = f.muu[x2 + 1], muv0 = f.muv[x2], muv1 = f.muv[x2 + sj];
+  const double fy0 = f.msfvy[x2], fy1 = f.msfvy[x2 + sj], fx0 = f.msfux[x2], fx1 = f.msfux[x2 + 1];
+  const double cyi = 0.25 * c.rdy / msfty, cyt = H * c.rdy / msfty, cxi = 0.25 * c.rdx / msfty, cxt = H * c.rdx / msfty;
+  const double r60 = 1.0 / 60.0;
+  const idx_t bj = full ? rj : 0;
+  auto phb = [&](idx_t dj, int d, int k) {  // the base geopotential at (i + d, the row dj away, k)
+    return full ? at(f.phb.p, bj + dj + k * sk)[d] : f.phb.p[idx_t(k) * f.phb.sk];
+  };
+  auto wdwn = [&](int m, real ww1, real ww0, real p1, real p0, double b1, double b0) {
+    return H * (ww1 + ww0) * c.rdnw[m] * (p1 - p0 + b1 - b0);
+  };
+  // the level below ka
+  const idx_t rm = rj + (ka - 1) * sk;
+  real q0 = at(ph, rm + sk)[0], ww0 = at(f.ww, rm + sk)[0];
+  real um0 = at(u, rm)[0], um1 = at(u, rm)[1], vm0 = at(v, rm)[0], vm1 = at(v, rm + sj)[0];
+  double b0 = phb(0, 0, ka);
+  double wd_m = wdwn(ka - 1, ww0, at(f.ww, rm)[0], q0, at(ph, rm)[0], b0, phb(0, 0, ka - 1));
+  for (int k = ka; k < kb; ++k) {
+    const idx_t r0 = rj + k * sk, rp = k < nz ? r0 + sk : r0;
+    const real* px = at(ph, r0);
+    const real xm3 = px[-3], xm2 = px[-2], xm1 = px[-1], xp1 = px[1], xp2 = px[2], xp3 = px[3];
+    const real ym3 = at(ph, r0 - 3 * sj)[0], ym2 = at(ph, r0 - 2 * sj)[0], ym1 = at(ph, r0 - sj)[0];
+    const real yp1 = at(ph, r0 + sj)[0], yp2 = at(ph, r0 + 2 * sj)[0], yp3 = at(ph, r0 + 3 * sj)[0];
+    const real qp = at(ph, rp)[0], wwp = at(f.ww, rp)[0], w = at(f.w2, r0)[0];
+    const real u0 = at(u, r0)[0], u1 = at(u, r0)[1], v0 = at(v, r0)[0], v1 = at(v, r0 + sj)[0];
+    const real hk = at(sp ? f.ph_tendf : ph, r0)[0];
+    const double bp = phb(0, 0, k < nz ? k + 1 : k);
+    // the base state's differences (0 where it is a profile)
+    double bx1 = 0, bx2 = 0, bx3 = 0, by1 = 0, by2 = 0, by3 = 0, bxc = 0, bxm = 0, bxp = 0;
+    if (full) {
+      const double* bx = at(f.phb.p, bj + k * sk);
+      bxm = bx[-1];
+      bxp = bx[1];
+      bxc = bx[0];
+      bx1 = bxp - bxm;
+      bx2 = bx[2] - bx[-2];
+      bx3 = bx[3] - bx[-3];
+      by1 = phb(sj, 0, k) - phb(-sj, 0, k);
+      by2 = phb(2 * sj, 0, k) - phb(-2 * sj, 0, k);
+      by3 = phb(3 * sj, 0, k) - phb(-3 * sj, 0, k);
+    }
+    double t = 0, wd = 0;
+    if (k < nz) {
+      wd = wdwn(k, wwp, ww0, qp, q0, bp, b0);
+      t = t - (c.fnm[k] * wd + c.fnp[k] * wd_m);
+    }
+    t = t + (c.c1f[k] * mut + c.c2f[k]) * kG * w / msfty;
+    // at the lid the winds are extrapolated from levels nz - 1, nz - 2
+    const idx_t r1 = r0 - sk, r2 = k < nz ? r1 : r1 - sk;
+    if (!two_d) {
+      const double mvp = c.c1f[k] * muv1 + c.c2f[k], mvm = c.c1f[k] * muv0 + c.c2f[k];
+      const double vp = k < nz ? v1 + vm1 : c.cfn * vm1 + c.cfn1 * at(v, r2 + sj)[0];
+      const double vm = k < nz ? v0 + vm0 : c.cfn * vm0 + c.cfn1 * at(v, r2)[0];
+      const double gy = 45.0 * (yp1 - ym1) - 9.0 * (yp2 - ym2) + (yp3 - ym3) + 45.0 * by1 - 9.0 * by2 + by3;
+      t = t - (k < nz ? cyi : cyt) * ((mvp * vp * fy1 + mvm * vm * fy0) * r60 * gy);
+    }
+    const double mup = c.c1f[k] * muu1 + c.c2f[k], mum = c.c1f[k] * muu0 + c.c2f[k];
+    const double up = k < nz ? u1 + um1 : c.cfn * um1 + c.cfn1 * at(u, r2)[1];
+    const double um = k < nz ? u0 + um0 : c.cfn * um0 + c.cfn1 * at(u, r2)[0];
+    const double cx = k < nz ? cxi : cxt;
+    const double gx = 45.0 * (xp1 - xm1) - 9.0 * (xp2 - xm2) + (xp3 - xm3) + 45.0 * bx1 - 9.0 * bx2 + bx3;
+    const double t6 = t - cx * ((mup * up * fx1 + mum * um * fx0) * r60 * gx);
+    if (xin) {
+      t = t6;
+    } else {  // one-sided differences on the column next to the edge's
+      const double de = bxp - bxc + xp1 - q0, dw = bxc - bxm + q0 - xm1;
+      const double t2 = t - cx * (mup * up * fx1 * de + mum * um * fx0 * dw);
+      t = ox == 6 ? t6 : (ox == 2 ? t2 : t);
+    }
+    if (sp) t = t + hk / msfty;  // rk_addtend_dry with a LateralBC (large_step.cpp:663)
+    row_st(f.ph_tend, r0, at.eo, t);
+    wd_m = wd;
+    q0 = qp;
+    ww0 = wwp;
+    b0 = bp;
+    um0 = u0; um1 = u1; vm0 = v0; vm1 = v1;
+  }
+}
+template <bool OPEN>
+MI_POINT_KERNEL k_tend_ph(Range r, int lv, Args a) {
+  const Piece pc = level_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  if (!pc.on) return;
+  const Geo& g = a.g;
+  const Fields& f = a.f;
+  const Lv& c = a.c;
+  const int i = pc.i, j = pc.j;
+  if (!OPEN && (!g.fly() || (j >= 3 && j < g.ny - 3))) {  // the rows with the 6th-order y gradient
+    tend_ph_levels(a, i, j, pc.ka, pc.kb);
+    return;
+  }
+  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
   const int nz = g.nz;
   const idx_t sj = g.sj, sk = g.sk;
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
@@ -1531,6 +1631,7 @@ MI_POINT_KERNEL k_tend_ph(Range r, Args a) {
   }
   if (sp) t = t + f.ph_tendf[x] / msfty;  // rk_addtend_dry with a LateralBC (large_step.cpp:663)
   f.ph_tend[x] = t;
+  }
 }
 
 // a / b in the substep kernels: the IEEE division in FP64 (the reference's bits); in FP32-bulk a multiply by the
@@ -1567,60 +1668,70 @@ __device__ __forceinline__ double damp_weight(const Args& a, int i, int j, int k
 
 // ----------------------------------------------------------------------------- small_step_prep
 // KPrep (reference src/dyn/small_step.cpp:39-93)
-MI_POINT_KERNEL k_ss_prep(Range r, Args a, int first) {
-  MI_POINT_INDEX(r)
+// A level piece per thread: the 2-D masses and map factors are read once, a level's 15 loads are issued together.
+// Bounded by its 17 stores per point: 425x300x50 FP32-bulk 229 -> 199 us per launch, 3.5 TB/s of its 27 arrays.
+MI_POINT_KERNEL k_ss_prep(Range r, int lv, Args a, int first) {
+  const Piece pc = level_piece(r, lv);
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
-  const double mts = f.mub[x2] + f.mu1[x2];
-  const double mus_u = first ? f.muu[x2] : H * (mts + f.mub[x2 - 1] + f.mu1[x2 - 1]);
-  const double mus_v = first ? f.muv[x2] : H * (mts + f.mub[x2 - g.sj] + f.mu1[x2 - g.sj]);
-  if (k == 0) {
+  const int i = pc.i, j = pc.j, nx = g.nx, ny = g.ny, nz = g.nz;
+  const idx_t x2 = g.at2(i, j), rj = j * g.sj - kLpad;
+  const Row at = row_of(i);
+  const double mts = f.mub[x2] + f.mu1[x2], muu = f.muu[x2], muv = f.muv[x2], mut = f.mut[x2];
+  const double mus_u = first ? muu : H * (mts + f.mub[x2 - 1] + f.mu1[x2 - 1]);
+  const double mus_v = first ? muv : H * (mts + f.mub[x2 - g.sj] + f.mu1[x2 - g.sj]);
+  const double msfuy = f.msfuy[x2], mvi = f.msfvx_inv[x2], msfty = f.msfty[x2];
+  const bool mass = i < nx && j < ny;
+  if (pc.ka == 0) {
     // the map-factor ratios advance_uv reads at every substep: msfux / msfuy, 1 / msfuy (u faces), msfvy / msfvx
     // (v faces)
     if (j < ny) {
-      f.rmu[x2] = f.msfux[x2] / f.msfuy[x2];
-      f.msfuy_inv[x2] = 1.0 / f.msfuy[x2];
+      f.rmu[x2] = f.msfux[x2] / msfuy;
+      f.msfuy_inv[x2] = 1.0 / msfuy;
     }
     if (i < nx && j < g.nyv) f.rmv[x2] = f.msfvy[x2] / f.msfvx[x2];
-    if (i < nx && j < ny) f.msfty_inv[x2] = 1.0 / f.msfty[x2];  // and the substeps' 1 / msfty
-    if (i < nx && j < ny) {
-      put<kHMass>(f.muts, g, i, j, 0, mts);
+    if (mass) f.msfty_inv[x2] = 1.0 / msfty;  // and the substeps' 1 / msfty
+    if (mass) {
+      f.muts[x2] = mts;
       const double m2 = f.mu2[x2];
       f.mu_save[x2] = m2;
-      put<kHMass>(f.mu2, g, i, j, 0, f.mu1[x2] - m2);
+      f.mu2[x2] = f.mu1[x2] - m2;
     }
     if (j < ny) f.muus[x2] = mus_u;
     if (i < nx && j < g.nyv) f.muvs[x2] = mus_v;
   }
-  if (j < ny && k < nz) {
-    const double ui = f.u2[x];
-    put<kHU>(f.u_save, g, i, j, k * g.sk, ui);
-    // the substeps' coupled save (mass x u_save / msfuy), constant within the stage
-    f.ucs[x] = bdiv((c.c1h[k] * f.muu[x2] + c.c2h[k]) * double(f.u_save[x]), f.msfuy[x2]);
-    put<kHU>(f.u2, g, i, j, k * g.sk, ((c.c1h[k] * mus_u + c.c2h[k]) * f.u1[x] - (c.c1h[k] * f.muu[x2] + c.c2h[k]) * ui) / f.msfuy[x2]);
-  }
-  if (i < nx && j < g.nyv && k < nz) {
-    const double vi = f.v2[x];
-    put<kHV>(f.v_save, g, i, j, k * g.sk, vi);
-    f.vcs[x] = (c.c1h[k] * f.muv[x2] + c.c2h[k]) * double(f.v_save[x]) * f.msfvx_inv[x2];
-    put<kHV>(f.v2, g, i, j, k * g.sk, ((c.c1h[k] * mus_v + c.c2h[k]) * f.v1[x] - (c.c1h[k] * f.muv[x2] + c.c2h[k]) * vi) * f.msfvx_inv[x2]);
-  }
-  if (i < nx && j < ny) {
-    if (k < nz) {
-      const double ti = f.t2[x];
-      put<kHMass>(f.t_save, g, i, j, k * g.sk, ti);
-      f.t2[x] = (c.c1h[k] * mts + c.c2h[k]) * f.t1[x] - (c.c1h[k] * f.mut[x2] + c.c2h[k]) * ti;
-      f.c2a[x] = kCpovcv * (f.pb(i, j, k) + f.p[x]) / f.alt[x];
+  for (int k = pc.ka; k < pc.kb; ++k) {
+    const idx_t r0 = rj + k * g.sk;
+    const real ui = at(f.u2, r0)[0], u1 = at(f.u1, r0)[0], vi = at(f.v2, r0)[0], v1 = at(f.v1, r0)[0];
+    const real ti = at(f.t2, r0)[0], t1 = at(f.t1, r0)[0], p = at(f.p, r0)[0], alt = at(f.alt, r0)[0];
+    const real wi = at(f.w2, r0)[0], w1 = at(f.w1, r0)[0], phi = at(f.ph2, r0)[0], ph1 = at(f.ph1, r0)[0], ww = at(f.ww, r0)[0];
+    const double pb = f.pb.si ? row_ld(f.pb.p, r0, at.eo) : f.pb.p[idx_t(k) * f.pb.sk];
+    const double c1h = c.c1h[k < nz ? k : 0], c2h = c.c2h[k < nz ? k : 0], c1f = c.c1f[k], c2f = c.c2f[k];
+    if (j < ny && k < nz) {
+      row_st(f.u_save, r0, at.eo, ui);
+      // the substeps' coupled save (mass x u_save / msfuy), constant within the stage
+      row_st(f.ucs, r0, at.eo, bdiv((c1h * muu + c2h) * double(ui), msfuy));
+      row_st(f.u2, r0, at.eo, ((c1h * mus_u + c2h) * u1 - (c1h * muu + c2h) * double(ui)) / msfuy);
     }
-    const double wi = f.w2[x], phi = f.ph2[x];
-    f.w_save[x] = wi;
-    f.w2[x] = ((c.c1f[k] * mts + c.c2f[k]) * f.w1[x] - (c.c1f[k] * f.mut[x2] + c.c2f[k]) * wi) / f.msfty[x2];
-    f.ph_save[x] = phi;
-    put<kHMass>(f.ph2, g, i, j, k * g.sk, f.ph1[x] - phi);
-    f.ww1[x] = (k == 0 || k == nz) ? 0.0 : f.ww[x];
+    if (i < nx && j < g.nyv && k < nz) {
+      row_st(f.v_save, r0, at.eo, vi);
+      row_st(f.vcs, r0, at.eo, (c1h * muv + c2h) * double(vi) * mvi);
+      row_st(f.v2, r0, at.eo, ((c1h * mus_v + c2h) * v1 - (c1h * muv + c2h) * double(vi)) * mvi);
+    }
+    if (mass) {
+      if (k < nz) {
+        row_st(f.t_save, r0, at.eo, ti);
+        row_st(f.t2, r0, at.eo, (c1h * mts + c2h) * t1 - (c1h * mut + c2h) * double(ti));
+        row_st(f.c2a, r0, at.eo, kCpovcv * (pb + p) / alt);
+      }
+      row_st(f.w_save, r0, at.eo, wi);
+      row_st(f.w2, r0, at.eo, ((c1f * mts + c2f) * w1 - (c1f * mut + c2f) * double(wi)) / msfty);
+      row_st(f.ph_save, r0, at.eo, phi);
+      row_st(f.ph2, r0, at.eo, ph1 - double(phi));
+      row_st(f.ww1, r0, at.eo, (k == 0 || k == nz) ? 0.0 : double(ww));
+    }
   }
 }
 
@@ -4712,12 +4823,12 @@ void launch_tendencies(const Args& a, hipStream_t st) {
   go("tend_t", op ? (a.f.thf ? k_tend_t<true, true> : k_tend_t<true, false>)
                   : (a.f.thf ? k_tend_t<false, true> : k_tend_t<false, false>),
      Range{0, g.nx, 0, g.ny, 0, g.nz});
-  launch3("tend_ph", op ? k_tend_ph<true> : k_tend_ph<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1}, st, a);
+  go("tend_ph", op ? k_tend_ph<true> : k_tend_ph<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1});
 }
 
 void launch_ss_prep(const Args& a, bool first, hipStream_t st) {
   const Geo& g = a.g;
-  launch3("ss_prep", k_ss_prep, Range{0, g.nx + 1, 0, g.nyv, 0, g.nz + 1}, st, a, first ? 1 : 0);
+  launch_pieces("ss_prep", point_bytes("ss_prep"), k_ss_prep, Range{0, g.nx + 1, 0, g.nyv, 0, g.nz + 1}, st, a, first ? 1 : 0);
 }
 void launch_ss_column(const Args& a, int cfg, double cof, double dts, hipStream_t st) {
   dispatch_cfg<SsColumnL>(cfg, "ss_column", 3, 0, a.g.nx, a.g.ny, st, a, cof, dts);
