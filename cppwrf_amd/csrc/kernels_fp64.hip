@@ -418,6 +418,51 @@ constexpr int kChain = 8;
 #define MI_COLUMN_KERNEL template <int CI, int KT> __global__ void __launch_bounds__(CI * KT)
 #define LDS(arr, k, ci) (arr)[(k) * CI + (ci)]
 
+// ----------------------------------------------------------------------------- level pieces
+// A wavefront's view of the fields: 64 consecutive points of one row (j and k are the same for all its lanes), so an
+// access is a scalar row address + the lane's 32-bit offset from the row's start (8 points west of i = 0).
+template <class T>
+__device__ __forceinline__ T row_ld(const T* p, idx_t row, unsigned eo) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ void row_st(T* p, idx_t row, unsigned eo, double v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(p + row) + eo * unsigned(sizeof(T))) = T(v);
+}
+
+// A block of the level-piece kernels: 64 points of four rows (a wavefront per row) x lv levels; the block grid is
+// x tiles, y tiles, level pieces, dealt to the XCDs in eighths, the pieces of a tile back to back (point_block)
+struct Piece {
+  int i, j, ka, kb;
+  bool on;
+};
+__device__ __forceinline__ Piece level_piece(const Range& r, int lv) {
+  const Blk b = point_block(1);
+  Piece p;
+  p.i = r.i0 + b.x * kBx + int(threadIdx.x);
+  p.j = r.j0 + b.y * int(blockDim.y) + __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+  p.ka = r.k0 + b.z * lv;
+  p.kb = p.ka + lv < r.k1 ? p.ka + lv : r.k1;
+  p.on = p.i < r.i1 && p.j < r.j1;
+  return p;
+}
+struct Row {  // the row's accessors: p[d] at (i + d) of the row that starts at index row
+  unsigned eo;
+  template <class T>
+  __device__ __forceinline__ const T* operator()(const T* p, idx_t row) const {
+    return reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
+  }
+};
+__device__ __forceinline__ Row row_of(int i) {
+  unsigned eo = unsigned(kLpad + i);
+  asm("" : "+v"(eo));
+  return Row{eo};
+}
+// a column kernel's level index: with 64 columns per block a wavefront holds one level, known to be uniform
+template <int CI>
+__device__ __forceinline__ int col_level(int kt) {
+  return CI == 64 ? __builtin_amdgcn_readfirstlane(kt) : kt;
+}
 // ----------------------------------------------------------------------------- rk_step_prep
 // One kernel over the (nx+1) x nyv columns of the U/V/W points (reference LargeStep::prep,
 // large_step.cpp:697-733, without its halo exchanges, none of which these kernels read):
@@ -425,6 +470,8 @@ constexpr int kChain = 8;
 //         by the others with the same expression (identical values)
 //   KPrep3 couple_momentum, calc_alt, calc_php (large_step.cpp:68-81)
 //   KWW   calc_ww_cp (large_step.cpp:83-108): divergence in parallel, the sums in k order from LDS
+// Bound by the latency of its reads: the 2-D fields are read once per column and a level's loads are issued together from
+// scalar row addresses (425x300x50 FP32-bulk, 64 columns x 4 levels: 204 -> 135 us a launch).
 MI_COLUMN_KERNEL k_large_prep(Args a) {
   constexpr int kKT = KT;
   extern __shared__ double lds[];
@@ -464,20 +511,39 @@ MI_COLUMN_KERNEL k_large_prep(Args a) {
     const double mu0 = mass ? H * (mu(i, j) + mub(i, j) + mu(i - 1, j) + mub(i - 1, j)) : 0.0;
     const double mv1 = mass ? H * (mu(i, j + 1) + mub(i, j + 1) + mu(i, j) + mub(i, j)) : 0.0;
     const double mv0 = mass ? H * (mu(i, j) + mub(i, j) + mu(i, j - 1) + mub(i, j - 1)) : 0.0;
-    for (int k = cp.kt; k <= nz; k += kKT) {
-      const idx_t x = g.at(i, j, k);
-      if (j < ny && k < nz) put<kHU>(f.ru, g, i, j, k * g.sk, f.u2[x] * (c.c1h[k] * muu + c.c2h[k]) / f.msfuy[x2]);
-      if (i < nx && j < g.nyv && k < nz) put<kHV>(f.rv, g, i, j, k * g.sk, f.v2[x] * (c.c1h[k] * muv + c.c2h[k]) * f.msfvx_inv[x2]);
+    // the 2-D fields read once (the stores below may alias them as far as the compiler knows), a level's loads together
+    const double mfy0 = f.msfuy[x2], mfy1 = f.msfuy[x2 + 1], mvi0 = f.msfvx_inv[x2], mvi1 = f.msfvx_inv[x2 + g.sj];
+    const double mty = f.msfty[x2], mtx = f.msftx[x2];
+    const idx_t rj = j * g.sj - kLpad, sk = g.sk;
+    const unsigned eo = unsigned(kLpad + i);
+    const bool full = f.alb.si != 0, uon = j < ny, von = i < nx && j < g.nyv;
+    for (int k = col_level<CI>(cp.kt); k <= nz; k += kKT) {
+      const idx_t r = rj + k * sk, rp = k < nz ? r + sk : r;
+      const int kc = k < nz ? k : nz - 1, kp = k < nz ? k + 1 : k;
+      const real u0 = row_ld(f.u2, r, eo), u1 = row_ld(f.u2, r, eo + 1u), v0 = row_ld(f.v2, r, eo), v1 = row_ld(f.v2, r + g.sj, eo);
+      const real w0 = row_ld(f.w2, r, eo), al = row_ld(f.al, r, eo), h0 = row_ld(f.ph2, r, eo), h1 = row_ld(f.ph2, rp, eo);
+      double alb, b0, b1;
+      if (full) {
+        alb = row_ld(f.alb.p, r, eo);
+        b0 = row_ld(f.phb.p, r, eo);
+        b1 = row_ld(f.phb.p, rp, eo);
+      } else {
+        alb = f.alb.p[idx_t(kc) * f.alb.sk];
+        b0 = f.phb.p[idx_t(k) * f.phb.sk];
+        b1 = f.phb.p[idx_t(kp) * f.phb.sk];
+      }
+      const double c1h = c.c1h[kc], c2h = c.c2h[kc];
+      if (uon && k < nz) row_st(f.ru, r, eo, u0 * (c1h * muu + c2h) / mfy0);
+      if (von && k < nz) row_st(f.rv, r, eo, v0 * (c1h * muv + c2h) * mvi0);
       if (mass) {
-        put<kHMass>(f.rw, g, i, j, k * g.sk, f.w2[x] * (c.c1f[k] * mut + c.c2f[k]) / f.msfty[x2]);
+        row_st(f.rw, r, eo, w0 * (c.c1f[k] * mut + c.c2f[k]) / mty);
         if (k < nz) {
-          put<kHMass>(f.alt, g, i, j, k * g.sk, f.al[x] + f.alb(i, j, k));
-          put<kHMass>(f.php, g, i, j, k * g.sk, H * (f.phb(i, j, k) + f.phb(i, j, k + 1) + f.ph2[x] + f.ph2[x + g.sk]));
+          row_st(f.alt, r, eo, al + alb);
+          row_st(f.php, r, eo, H * (b0 + b1 + h0 + h1));
           LDS(dv, k, cp.ci) =
-              f.msftx[x2] * c.dnw[k] *
-              (c.rdx * ((c.c1h[k] * mu1 + c.c2h[k]) * f.u2[x + 1] / f.msfuy[x2 + 1] - (c.c1h[k] * mu0 + c.c2h[k]) * f.u2[x] / f.msfuy[x2]) +
-               c.rdy * ((c.c1h[k] * mv1 + c.c2h[k]) * f.v2[x + g.sj] * f.msfvx_inv[x2 + g.sj] -
-                        (c.c1h[k] * mv0 + c.c2h[k]) * f.v2[x] * f.msfvx_inv[x2]));
+              mtx * c.dnw[k] *
+              (c.rdx * ((c1h * mu1 + c2h) * u1 / mfy1 - (c1h * mu0 + c2h) * u0 / mfy0) +
+               c.rdy * ((c1h * mv1 + c2h) * v1 * mvi1 - (c1h * mv0 + c2h) * v0 * mvi0));
         }
       }
     }
@@ -515,34 +581,6 @@ MI_COLUMN_KERNEL k_large_prep(Args a) {
   }
 }
 
-// ----------------------------------------------------------------------------- level pieces
-// A wavefront's view of the fields: 64 consecutive points of one row (j and k are the same for all its lanes), so an
-// access is a scalar row address + the lane's 32-bit offset from the row's start (8 points west of i = 0).
-template <class T>
-__device__ __forceinline__ T row_ld(const T* p, idx_t row, unsigned eo) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
-}
-template <class T>
-__device__ __forceinline__ void row_st(T* p, idx_t row, unsigned eo, double v) {
-  *reinterpret_cast<T*>(reinterpret_cast<char*>(p + row) + eo * unsigned(sizeof(T))) = T(v);
-}
-
-// A block of the level-piece kernels: 64 points of four rows (a wavefront per row) x lv levels; the block grid is
-// x tiles, y tiles, level pieces, dealt to the XCDs in eighths, the pieces of a tile back to back (point_block)
-struct Piece {
-  int i, j, ka, kb;
-  bool on;
-};
-__device__ __forceinline__ Piece level_piece(const Range& r, int lv) {
-  const Blk b = point_block(1);
-  Piece p;
-  p.i = r.i0 + b.x * kBx + int(threadIdx.x);
-  p.j = r.j0 + b.y * int(blockDim.y) + __builtin_amdgcn_readfirstlane(int(threadIdx.y));
-  p.ka = r.k0 + b.z * lv;
-  p.kb = p.ka + lv < r.k1 ? p.ka + lv : r.k1;
-  p.on = p.i < r.i1 && p.j < r.j1;
-  return p;
-}
 // ----------------------------------------------------------------------------- rk_tendency
 // KTendU (large_step.cpp:152-264): advect_u + horizontal pressure gradient + curvature, interior faces
 // MapC::vxgm (large_step.cpp:121-124): the map-factor curvature term at the mass point of index y (2-D y2)
@@ -609,18 +647,6 @@ __device__ __forceinline__ double open_y_scalar(const Geo& g, const T* q, const 
 // the per-level kernels' below, operand for operand; the marches take the rows whose y fluxes have the domain's own
 // order and the wavefronts without an open edge, the per-level code the others.  Columns next to a specified or open x
 // side pick their x flux's order lane by lane.
-struct Row {  // the row's accessors: p[d] at (i + d) of the row that starts at index row
-  unsigned eo;
-  template <class T>
-  __device__ __forceinline__ const T* operator()(const T* p, idx_t row) const {
-    return reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
-  }
-};
-__device__ __forceinline__ Row row_of(int i) {
-  unsigned eo = unsigned(kLpad + i);
-  asm("" : "+v"(eo));
-  return Row{eo};
-}
 // KTendU (DIR 0) and KTendV (DIR 1): the same terms with the two directions exchanged
 template <int DIR>
 __device__ __forceinline__ void tend_uv_levels(const Args& a, int i, int j, int ka, int kb) {
@@ -3000,7 +3026,8 @@ __global__ void __launch_bounds__(KT) k_acoustic_ring(Args a, double dts, int it
 // ----------------------------------------------------------------------------- small_step_finish
 // KFinish + KFinishMu (small_step.cpp:419-454) over the (nx+1) x nyv columns and, with prhophi set,
 // calc_p_rho_phi (KPRhoPhi, small_step.cpp:456-477) of the mass columns from the recoupled state: the
-// reference refreshes halos in between, which KPRhoPhi does not read.
+// reference refreshes halos in between, which KPRhoPhi does not read.  Laid out as k_large_prep (425x300x50 FP32-bulk: 235 ->
+// 185 us a launch).
 MI_COLUMN_KERNEL k_finish(Args a, int prhophi, double hd_dt) {
   constexpr int kKT = KT;
   extern __shared__ double lds[];
@@ -3019,19 +3046,28 @@ MI_COLUMN_KERNEL k_finish(Args a, int prhophi, double hd_dt) {
     const double mus_u = j < ny ? H * (muts + f.muts[x2 - 1]) : 0.0;
     const double mus_v = (i < nx && j < g.nyv) ? H * (muts + f.muts[x2 - g.sj]) : 0.0;
     const double m = mass ? f.mut[x2] : 0.0;
-    for (int k = cp.kt; k <= nz; k += kKT) {
-      const idx_t x = g.at(i, j, k);
-      if (j < ny && k < nz)
-        put<kHU>(f.u2, g, i, j, k * g.sk, (f.msfuy[x2] * f.u2[x] + f.u_save[x] * (c.c1h[k] * f.muu[x2] + c.c2h[k])) / (c.c1h[k] * mus_u + c.c2h[k]));
-      if (i < nx && j < g.nyv && k < nz)
-        put<kHV>(f.v2, g, i, j, k * g.sk, (f.msfvx[x2] * f.v2[x] + f.v_save[x] * (c.c1h[k] * f.muv[x2] + c.c2h[k])) / (c.c1h[k] * mus_v + c.c2h[k]));
+    const double mfy = f.msfuy[x2], mvx = f.msfvx[x2], mty = f.msfty[x2], muu = f.muu[x2], muv = f.muv[x2];
+    const idx_t rj = j * g.sj - kLpad, sk = g.sk;
+    const unsigned eo = unsigned(kLpad + i);
+    const bool heat = hd_dt != 0.0, uon = j < ny, von = i < nx && j < g.nyv;
+    for (int k = col_level<CI>(cp.kt); k <= nz; k += kKT) {
+      const idx_t r = rj + k * sk;
+      // a level's loads together, none conditional
+      const real u = row_ld(f.u2, r, eo), us = row_ld(f.u_save, r, eo), v = row_ld(f.v2, r, eo), vs = row_ld(f.v_save, r, eo);
+      const real w = row_ld(f.w2, r, eo), ws = row_ld(f.w_save, r, eo), h = row_ld(f.ph2, r, eo), hs = row_ld(f.ph_save, r, eo);
+      const real ww = row_ld(f.ww, r, eo), w1 = row_ld(f.ww1, r, eo), t = row_ld(f.t2, r, eo), ts = row_ld(f.t_save, r, eo);
+      const real hd = row_ld(heat ? f.hdia : f.t2, r, eo);
+      const int kc = k < nz ? k : nz - 1;
+      const double c1h = c.c1h[kc], c2h = c.c2h[kc], c1f = c.c1f[k], c2f = c.c2f[k];
+      if (uon && k < nz) row_st(f.u2, r, eo, (mfy * u + us * (c1h * muu + c2h)) / (c1h * mus_u + c2h));
+      if (von && k < nz) row_st(f.v2, r, eo, (mvx * v + vs * (c1h * muv + c2h)) / (c1h * mus_v + c2h));
       if (mass) {
-        put<kHMass>(f.w2, g, i, j, k * g.sk, (f.msfty[x2] * f.w2[x] + f.w_save[x] * (c.c1f[k] * m + c.c2f[k])) / (c.c1f[k] * muts + c.c2f[k]));
-        const double phk = f.ph2[x] + f.ph_save[x];
-        put<kHMass>(f.ph2, g, i, j, k * g.sk, phk);
+        row_st(f.w2, r, eo, (mty * w + ws * (c1f * m + c2f)) / (c1f * muts + c2f));
+        const double phk = h + hs;
+        row_st(f.ph2, r, eo, phk);
         LDS(PH, k, ci) = double(real(phk));  // the value as stored (the same as calc_p_rho_phi reads alone)
-        put<kHMass>(f.ww, g, i, j, k * g.sk, f.ww[x] + f.ww1[x]);
-        if (k < nz) put<kHMass>(f.t2, g, i, j, k * g.sk, (f.t2[x] - (hd_dt != 0.0 ? hd_dt * (c.c1h[k] * m + c.c2h[k]) * f.hdia[x] : 0.0) + f.t_save[x] * (c.c1h[k] * m + c.c2h[k])) / (c.c1h[k] * muts + c.c2h[k]));
+        row_st(f.ww, r, eo, ww + w1);
+        if (k < nz) row_st(f.t2, r, eo, (t - (heat ? hd_dt * (c1h * m + c2h) * hd : 0.0) + ts * (c1h * m + c2h)) / (c1h * muts + c2h));
       }
     }
     if (cp.kt == 0) {
@@ -4784,7 +4820,9 @@ bool col_cfg_fits(int kernel, int cfg, int nz) {
 
 int col_cfg_default(int kernel, int nx, int ny, int nz) {
   // the substep kernel: the narrowest one-level-per-thread shape; the others: one level per thread on
-  // small domains (latency), 16 columns (full 128-byte rows) on larger ones
+  // small domains (latency); on larger ones 64 columns x 4 levels, a wavefront a row, where the work is the loads and
+  // stores (large_prep, finish: 425x300x50 12.42 -> 12.02 ms a step FP32-bulk, 21.1 -> 20.6 ms FP64, with the kernels'
+  // loads grouped), 16 columns x 16 for the ss column, whose sums over the levels need the narrower block's LDS
   if (kernel == kColAcoustic) {
     // FP32-bulk: several levels per thread (425x300x50 557 -> 446 us; FP64 is slower that way, 704 -> 775 us)
     if (kAcFp32) return kColLevels;
@@ -4793,7 +4831,7 @@ int col_cfg_default(int kernel, int nx, int ny, int nz) {
     return 6;
   }
   const bool small = int64_t(nx) * ny <= 16384;
-  const int pref[] = {small ? (nz + 1 <= 64 ? 4 : (nz + 1 <= 128 ? 5 : 6)) : 0, 3, 5, 6};
+  const int pref[] = {small ? (nz + 1 <= 64 ? 4 : (nz + 1 <= 128 ? 5 : 6)) : (kernel == kColSsColumn ? 0 : 7), 0, 3, 5, 6};
   for (int c : pref)
     if (col_cfg_fits(kernel, c, nz)) return c;
   return 6;
