@@ -1,8 +1,8 @@
 // The domain object behind the C ABI: device memory of one forecast, the launch schedule of
 // RK3::step (reference src/dyn/rk3.cpp:86-170) and its capture as a HIP graph.
 //
-// The schedule keeps the reference's points of halo refresh exactly (every halo read returns what the
-// reference's halo holds at that moment), because the FP64 results must be bit-identical.  Adjacent
+// Every halo read returns what the reference's halo holds at that moment, because the FP64 results must be
+// bit-identical; a refresh whose halo no kernel reads before the next one is left out.  Adjacent
 // halo refreshes with no kernel between them are merged into one launch pair (x pass, then y pass):
 // every field's x pass still precedes its y pass, as the reference's batched fill (halo.cpp:133-190).
 #include <hip/hip_runtime.h>
@@ -272,7 +272,7 @@ struct Domain final : mi_domain {
 
   // SmallStep::run_stage (small_step.cpp:490-607); with prhophi, calc_p_rho_phi (small_step.cpp:609-617)
   // is fused into the finishing kernel.  In four parts, which a batch interleaves with its members' (ss_begin, then
-  // per substep advance_uv, the column kernel and after_acoustic, then ss_end).
+  // per substep advance_uv and the column kernel, then ss_end).
   //
   // No kernel between the stage's prologue and its end reads a halo point: the substep kernels reach their neighbour
   // columns through the lateral boundary condition (a periodic side's column n is column 0, a mirrored or copied one
@@ -287,8 +287,7 @@ struct Domain final : mi_domain {
     ss_begin(rk);
     for (int it = 1; it <= ns; ++it) {
       launch_uv(a, dts, stream());
-      launch_acoustic(a, colcfg[kColAcoustic], dts, it, ns, stream());
-      after_acoustic(rk, it);
+      launch_acoustic(a, colcfg[kColAcoustic], dts, it, ns, stream());  // the spec zone's columns included
     }
     ss_end(rk, prhophi);
   }
@@ -301,7 +300,7 @@ struct Domain final : mi_domain {
     const double cof_h = 0.5 * dts * kG * (1.0 + prm.epssm);
     launch_ss_column(a, colcfg[kColSsColumn], cof_h * cof_h, dts, st);
   }
-  // after the substep's column kernel: the spec zone's columns
+  // after a batch's column kernel (launch_acoustic does it for a domain alone): the spec zone's columns
   void after_acoustic(int rk, int it) {
     if (spec) launch_acoustic_ring(a, stage_dts(rk), it, stage_ns(rk), stream());
   }

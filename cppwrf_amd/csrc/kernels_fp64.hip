@@ -1997,6 +1997,145 @@ MI_POINT_KERNEL k_uv(Range r, int lv, Args a, double dts) {
   if (p.on) uv_levels<OPEN>(a, p.i, p.j, p.ka, p.kb, dts);
 }
 
+// ----------------------------------------------------------------------------- the spec zone's substep
+// One acoustic substep of the spec zone's columns with specified boundaries (a thread per level), in the reference's order (SmallStep::run_stage, small_step.cpp:548-593, with LateralBC's updates,
+// lateral_bc.cpp:356-387):
+//   KMuTCol's ring branch: omega'' left as it stands, summed into ww_m (small_step.cpp:214-220)
+//   KMuTPoint's ru_m, rv_m sums (theta'' not advanced there) and KSumEdge's east and north domain faces
+//   update_mu_t: theta'', mu'' and muts += dts * tendency
+//   spec_bdyupdate_ph (KUpdatePh): phi'' of every level from the stage masses; w waits for zero_grad_bdy
+//   KWPRho: p'', al'' with divergence damping
+// The interior columns do not read these columns within a substep (every acoustic kernel reads its own
+// column, and the spec zone's faces were advanced by k_uv before), so the two are independent.
+//
+// ring_column: column `col` of the spec zone, level k of the calling thread; PH: nz + 1 doubles of LDS of the column.  Every
+// thread of the block calls it (two barriers); a column index beyond the zone does nothing.
+__device__ __forceinline__ int ring_columns(const Geo& g) { return 2 * g.nx + 2 * (g.ny - 2); }
+__device__ __forceinline__ void ring_column(const Args& a, int col, int k, double* PH, double dts, int it, int ns) {
+  const Geo& g = a.g;
+  const Fields& f = a.f;
+  const Lv& c = a.c;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const bool in = col < ring_columns(g);
+  if (!in) col = 0;
+  int i, j;  // S row, N row, W column, E column
+  if (col < nx) {
+    i = col;
+    j = 0;
+  } else if ((col -= nx) < nx) {
+    i = col;
+    j = ny - 1;
+  } else if ((col -= nx) < ny - 2) {
+    i = 0;
+    j = 1 + col;
+  } else {
+    i = nx - 1;
+    j = 1 + col - (ny - 2);
+  }
+  const bool on = in && k <= nz, mk = in && k < nz;
+  const bool first = it == 1, last = it == ns;
+  const double rn = double(ns);
+  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j), x = g.at(i, j, k <= nz ? k : nz);
+  const double mu_old = f.mu2[x2], mtend = f.mu_tend[x2], muts_old = f.muts[x2];
+  double wwcur = 0, wwm = 0, ww1 = 0, ph = 0, phtend = 0, phs = 0;
+  double u0 = 0, us0 = 0, v0 = 0, vs0 = 0, rum = 0, rvm = 0, u1 = 0, us1 = 0, v1 = 0, vs1 = 0, rum1 = 0, rvm1 = 0;
+  double t2 = 0, ttend = 0, ts = 0, c2a = 0, alt = 0, pm1 = 0;
+  if (on) {
+    wwcur = f.ww[x];
+    if (!first) wwm = f.ww_m[x];
+    ww1 = f.ww1[x];
+    ph = f.ph2[x];
+    phtend = f.ph_tend[x];
+    phs = f.ph_save[x];
+    if (mk) {
+      u0 = f.u2[x];
+      us0 = f.u_save[x];
+      v0 = f.v2[x];
+      vs0 = f.v_save[x];
+      t2 = f.t2[x];
+      ttend = f.t_tend[x];
+      ts = f.t_save[x];
+      c2a = f.c2a[x];
+      alt = f.alt[x];
+      pm1 = f.pm1[x];
+      if (i == nx - 1) {
+        u1 = f.u2[x + 1];
+        us1 = f.u_save[x + 1];
+      }
+      if (j == ny - 1) {
+        v1 = f.v2[x + sj];
+        vs1 = f.v_save[x + sj];
+      }
+      if (!first) {
+        rum = f.ru_m[x];
+        rvm = f.rv_m[x];
+        if (i == nx - 1) rum1 = f.ru_m[x + 1];
+        if (j == ny - 1) rvm1 = f.rv_m[x + sj];
+      }
+    }
+  }
+  __syncthreads();  // every level has read mu'' and muts before they change
+  const double mu_new = mu_old + dts * mtend, muts = muts_old + dts * mtend;
+  if (in && k == 0) {
+    put<kHMass>(f.mu2, g, i, j, 0, mu_new);
+    put<kHMass>(f.muts, g, i, j, 0, muts);
+  }
+  double t2new = 0;
+  if (on) {
+    const double sw = (first ? 0.0 : wwm) + wwcur;
+    put<kHMass>(f.ww_m, g, i, j, k * sk, last ? sw / rn + ww1 : sw);
+    if (mk) {
+      const double muu0 = f.muu[x2], msfuy0 = f.msfuy[x2], muv0 = f.muv[x2], mvi0 = f.msfvx_inv[x2];
+      const double su = (first ? 0.0 : rum) + u0;
+      put<kHU>(f.ru_m, g, i, j, k * sk, last ? su / rn + (c.c1h[k] * muu0 + c.c2h[k]) * us0 / msfuy0 : su);
+      const double sv = (first ? 0.0 : rvm) + v0;
+      put<kHV>(f.rv_m, g, i, j, k * sk, last ? sv / rn + (c.c1h[k] * muv0 + c.c2h[k]) * vs0 * mvi0 : sv);
+      if (i == nx - 1) {
+        const double se = (first ? 0.0 : rum1) + u1;
+        put<kHU>(f.ru_m, g, i + 1, j, k * sk,
+                 last ? se / rn + (c.c1h[k] * f.muu[x2 + 1] + c.c2h[k]) * us1 / f.msfuy[x2 + 1] : se);
+      }
+      if (j == ny - 1) {
+        const double sn = (first ? 0.0 : rvm1) + v1;
+        put<kHV>(f.rv_m, g, i, j + 1, k * sk,
+                 last ? sn / rn + (c.c1h[k] * f.muv[x2 + sj] + c.c2h[k]) * vs1 * f.msfvx_inv[x2 + sj] : sn);
+      }
+      t2new = t2 + dts * ttend;
+      f.t2[x] = t2new;
+    }
+    const double mu_o = muts - dts * mtend;
+    const double m_old = c.c1f[k] * mu_o + c.c2f[k], m_new = c.c1f[k] * muts + c.c2f[k];
+    const double phk = ph * m_old / m_new + dts * phtend / m_new + phs * (m_old / m_new - 1.0);
+    put<kHMass>(f.ph2, g, i, j, k * sk, phk);
+    PH[k] = phk;
+  }
+  __syncthreads();
+  if (mk) {
+    const double m = c.c1h[k] * muts + c.c2h[k];
+    const double al = -((1. / m) * (alt * (c.c1h[k] * mu_new) + c.rdnw[k] * (PH[k + 1] - PH[k])));
+    put<kHMass>(f.al, g, i, j, k * sk, al);
+    double pp = c2a * (alt * (t2new - c.c1h[k] * mu_new * ts) / (m * (kT0 + ts)) - al);
+    const double ptmp = pp;
+    pp = pp + a.q.smdiv * (pp - pm1);
+    f.pm1[x] = ptmp;
+    put<kHMass>(f.p, g, i, j, k * sk, pp);
+  }
+}
+template <int KT>
+__global__ void __launch_bounds__(KT) k_acoustic_ring(Args a, double dts, int it, int ns) {
+  __shared__ double PH[KT + 1];
+  ring_column(a, int(blockIdx.x), int(threadIdx.x), PH, dts, it, ns);
+}
+// The spec zone in the interior's launch: with at most 64 levels the column kernels' extra blocks (rows b.y >= ny of the
+// block grid) take a column per wavefront.  The two sets of columns do not read one another's results, so the
+// zone needs no launch of its own (28 us of its own at 425x300x50, 8 us at 119x89x44, at every substep).
+__device__ __forceinline__ bool ring_blocks(const Args& a, const Blk& b, double* lds, double dts, int it, int ns) {
+  if (b.y < a.g.ny) return false;
+  const int w = int(threadIdx.x) / 64, nw = int(blockDim.x) / 64;
+  ring_column(a, ((b.y - a.g.ny) * int(gridDim.x) + b.x) * nw + w, int(threadIdx.x) % 64, lds + w * (a.g.nz + 1), dts, it, ns);
+  return true;
+}
+
 // ----------------------------------------------------------------------------- one acoustic substep's column work
 // FP32-bulk with 64 threads per column: the column recurrences run as wave-wide scans, one wavefront per column
 // (wave w of the block takes column w, lane k level k).  The sums then associate differently and the Thomas
@@ -2047,14 +2186,14 @@ __device__ __forceinline__ double wave_affine_scan(double p, double q, int lane)
 //   8  KWSolve's damp_opt 3 damping and phi'' (small_step.cpp:388-406), parallel over levels
 //   9  KWPRho (small_step.cpp:409-414)
 // With specified boundaries the spec zone's columns (Edge::mass, small_step.cpp:39-45) are skipped here and
-// advanced by k_acoustic_ring.
+// advanced by ring_column.
 template <int CI, int KT>
 __device__ __forceinline__ void acoustic_cols(const Args& a, const ColPos cp, double* lds, double dts, int it, int ns) {
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
   const int i = cp.i, j = cp.j, nz = g.nz, ci = cp.ci, k = cp.kt;
-  // with specified boundaries the spec zone's columns are left to k_acoustic_ring
+  // with specified boundaries the spec zone's columns are ring_column's
   const bool ring = g.bcx == MI_BC_SPECIFIED && (i == 0 || i == g.nx - 1 || j == 0 || j == g.ny - 1);
   const bool on = i < g.nx && k <= nz && !ring;
   const int L = (nz + 1) * CI;
@@ -2387,6 +2526,9 @@ __device__ __forceinline__ void acoustic_cols(const Args& a, const ColPos cp, do
 }
 MI_COLUMN_KERNEL k_acoustic(Args a, double dts, int it, int ns) {
   extern __shared__ double lds[];
+  if constexpr (KT == 64) {
+    if (ring_blocks(a, xcd_block(), lds, dts, it, ns)) return;
+  }
   acoustic_cols<CI, KT>(a, col_pos<CI>(), lds, dts, it, ns);
 }
 
@@ -2421,7 +2563,7 @@ __device__ __forceinline__ void acoustic_levels(const Args& a, int bx, int j, do
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const int ci = int(threadIdx.x) % CI, kt = int(threadIdx.x) / CI, KT = int(blockDim.x) / CI;
   const int i = bx * CI + ci, k0 = kt * LPT;
-  // with specified boundaries the spec zone's columns are left to k_acoustic_ring
+  // with specified boundaries the spec zone's columns are ring_column's
   const bool ring = g.bcx == MI_BC_SPECIFIED && (i == 0 || i == nx - 1 || j == 0 || j == ny - 1);
   const bool on = i < nx && !ring;
   const bool two_d = g.two_d, moist = a.q.moist != 0, first = it == 1, last = it == ns;
@@ -2829,6 +2971,9 @@ template <int CI, int LPT, bool SCAN>
 __global__ void __launch_bounds__(512, kAcFp32 ? 3 : 2) k_acoustic_levels(Args a, double dts, int it, int ns) {
   extern __shared__ double lds[];
   const Blk b = xcd_block();
+  if constexpr (SCAN) {
+    if (ring_blocks(a, b, lds, dts, it, ns)) return;
+  }
   acoustic_levels<CI, LPT, SCAN>(a, b.x, b.y, lds, dts, it, ns);
 }
 
@@ -2878,7 +3023,7 @@ __global__ void __launch_bounds__(CI * KT) k_acoustic_batch(const Args* as, cons
 
 // KSumEdge (small_step.cpp:279-290, 560-569) of an open direction, after each substep's column kernel: the east
 // (north) domain face is a real face, its time average summed as the faces of the columns (with specified
-// boundaries k_acoustic_ring does it).  ydir 0: faces i = nx of the last column; 1: faces j = ny of the last row.
+// boundaries ring_column does it).  ydir 0: faces i = nx of the last column; 1: faces j = ny of the last row.
 MI_POINT_KERNEL k_open_sum(Range r, Args a, int it, int ns, int ydir) {
   MI_POINT_INDEX(r)
   const Geo& g = a.g;
@@ -2897,129 +3042,6 @@ MI_POINT_KERNEL k_open_sum(Range r, Args a, int it, int ns, int ydir) {
     const real v1 = f.v2[y], vs1 = f.v_save[y];
     const double sn = (first ? 0.0 : double(f.rv_m[y])) + v1;
     put<kHV>(f.rv_m, g, i, j + 1, k * sk, last ? sn / rn + (c.c1h[k] * f.muv[y2] + c.c2h[k]) * vs1 * f.msfvx_inv[y2] : sn);
-  }
-}
-
-// ----------------------------------------------------------------------------- the spec zone's substep
-// One acoustic substep of the spec zone's columns with specified boundaries (a block per column, a thread per
-// level), in the reference's order (SmallStep::run_stage, small_step.cpp:548-593, with LateralBC's updates,
-// lateral_bc.cpp:356-387):
-//   KMuTCol's ring branch: omega'' left as it stands, summed into ww_m (small_step.cpp:214-220)
-//   KMuTPoint's ru_m, rv_m sums (theta'' not advanced there) and KSumEdge's east and north domain faces
-//   update_mu_t: theta'', mu'' and muts += dts * tendency
-//   spec_bdyupdate_ph (KUpdatePh): phi'' of every level from the stage masses; w waits for zero_grad_bdy
-//   KWPRho: p'', al'' with divergence damping
-// The interior columns do not read these columns within a substep (every acoustic kernel reads its own
-// column, and the spec zone's faces were advanced by k_uv before), so the two kernels are independent.
-template <int KT>
-__global__ void __launch_bounds__(KT) k_acoustic_ring(Args a, double dts, int it, int ns) {
-  __shared__ double PH[KT + 1];
-  const Geo& g = a.g;
-  const Fields& f = a.f;
-  const Lv& c = a.c;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  int col = int(blockIdx.x), i, j;  // S row, N row, W column, E column
-  if (col < nx) {
-    i = col;
-    j = 0;
-  } else if ((col -= nx) < nx) {
-    i = col;
-    j = ny - 1;
-  } else if ((col -= nx) < ny - 2) {
-    i = 0;
-    j = 1 + col;
-  } else {
-    i = nx - 1;
-    j = 1 + col - (ny - 2);
-  }
-  const int k = int(threadIdx.x);
-  const bool on = k <= nz, mk = k < nz;
-  const bool first = it == 1, last = it == ns;
-  const double rn = double(ns);
-  const idx_t sk = g.sk, sj = g.sj, x2 = g.at2(i, j), x = g.at(i, j, on ? k : nz);
-  const double mu_old = f.mu2[x2], mtend = f.mu_tend[x2], muts_old = f.muts[x2];
-  double wwcur = 0, wwm = 0, ww1 = 0, ph = 0, phtend = 0, phs = 0;
-  double u0 = 0, us0 = 0, v0 = 0, vs0 = 0, rum = 0, rvm = 0, u1 = 0, us1 = 0, v1 = 0, vs1 = 0, rum1 = 0, rvm1 = 0;
-  double t2 = 0, ttend = 0, ts = 0, c2a = 0, alt = 0, pm1 = 0;
-  if (on) {
-    wwcur = f.ww[x];
-    if (!first) wwm = f.ww_m[x];
-    ww1 = f.ww1[x];
-    ph = f.ph2[x];
-    phtend = f.ph_tend[x];
-    phs = f.ph_save[x];
-    if (mk) {
-      u0 = f.u2[x];
-      us0 = f.u_save[x];
-      v0 = f.v2[x];
-      vs0 = f.v_save[x];
-      t2 = f.t2[x];
-      ttend = f.t_tend[x];
-      ts = f.t_save[x];
-      c2a = f.c2a[x];
-      alt = f.alt[x];
-      pm1 = f.pm1[x];
-      if (i == nx - 1) {
-        u1 = f.u2[x + 1];
-        us1 = f.u_save[x + 1];
-      }
-      if (j == ny - 1) {
-        v1 = f.v2[x + sj];
-        vs1 = f.v_save[x + sj];
-      }
-      if (!first) {
-        rum = f.ru_m[x];
-        rvm = f.rv_m[x];
-        if (i == nx - 1) rum1 = f.ru_m[x + 1];
-        if (j == ny - 1) rvm1 = f.rv_m[x + sj];
-      }
-    }
-  }
-  __syncthreads();  // every level has read mu'' and muts before they change
-  const double mu_new = mu_old + dts * mtend, muts = muts_old + dts * mtend;
-  if (k == 0) {
-    put<kHMass>(f.mu2, g, i, j, 0, mu_new);
-    put<kHMass>(f.muts, g, i, j, 0, muts);
-  }
-  double t2new = 0;
-  if (on) {
-    const double sw = (first ? 0.0 : wwm) + wwcur;
-    put<kHMass>(f.ww_m, g, i, j, k * sk, last ? sw / rn + ww1 : sw);
-    if (mk) {
-      const double muu0 = f.muu[x2], msfuy0 = f.msfuy[x2], muv0 = f.muv[x2], mvi0 = f.msfvx_inv[x2];
-      const double su = (first ? 0.0 : rum) + u0;
-      put<kHU>(f.ru_m, g, i, j, k * sk, last ? su / rn + (c.c1h[k] * muu0 + c.c2h[k]) * us0 / msfuy0 : su);
-      const double sv = (first ? 0.0 : rvm) + v0;
-      put<kHV>(f.rv_m, g, i, j, k * sk, last ? sv / rn + (c.c1h[k] * muv0 + c.c2h[k]) * vs0 * mvi0 : sv);
-      if (i == nx - 1) {
-        const double se = (first ? 0.0 : rum1) + u1;
-        put<kHU>(f.ru_m, g, i + 1, j, k * sk,
-                 last ? se / rn + (c.c1h[k] * f.muu[x2 + 1] + c.c2h[k]) * us1 / f.msfuy[x2 + 1] : se);
-      }
-      if (j == ny - 1) {
-        const double sn = (first ? 0.0 : rvm1) + v1;
-        put<kHV>(f.rv_m, g, i, j + 1, k * sk,
-                 last ? sn / rn + (c.c1h[k] * f.muv[x2 + sj] + c.c2h[k]) * vs1 * f.msfvx_inv[x2 + sj] : sn);
-      }
-      t2new = t2 + dts * ttend;
-      f.t2[x] = t2new;
-    }
-    const double mu_o = muts - dts * mtend;
-    const double m_old = c.c1f[k] * mu_o + c.c2f[k], m_new = c.c1f[k] * muts + c.c2f[k];
-    const double phk = ph * m_old / m_new + dts * phtend / m_new + phs * (m_old / m_new - 1.0);
-    put<kHMass>(f.ph2, g, i, j, k * sk, phk);
-    PH[k] = phk;
-  }
-  __syncthreads();
-  if (mk) {
-    const double m = c.c1h[k] * muts + c.c2h[k];
-    const double al = -((1. / m) * (alt * (c.c1h[k] * mu_new) + c.rdnw[k] * (PH[k + 1] - PH[k])));
-    put<kHMass>(f.al, g, i, j, k * sk, al);
-    double pp = c2a * (alt * (t2new - c.c1h[k] * mu_new * ts) / (m * (kT0 + ts)) - al);
-    const double ptmp = pp;
-    pp = pp + a.q.smdiv * (pp - pm1);
-    f.pm1[x] = ptmp;
-    put<kHMass>(f.p, g, i, j, k * sk, pp);
   }
 }
 
@@ -4781,12 +4803,7 @@ void dispatch_cfg(int cfg, T&&... args) {
   }
 }
 
-// the points a column kernel advances: the substep kernel leaves the spec zone's columns to k_acoustic_ring
-double col_points(const char* name, const Args& a) {
-  double cols = double(a.g.nx) * double(a.g.ny);
-  if (a.g.bcx == MI_BC_SPECIFIED && std::strcmp(name, "acoustic") == 0) cols -= 2.0 * (a.g.nx + a.g.ny) - 4.0;
-  return cols * double(a.g.nz);
-}
+double col_points(const Args& a) { return double(a.g.nx) * double(a.g.ny) * double(a.g.nz); }
 
 // one launch of a column kernel with block shape (CI, KT), timed when selected
 #define MI_COL_LAUNCHER(Name, kern)                                                                              \
@@ -4800,19 +4817,34 @@ double col_points(const char* name, const Args& a) {
       if (t) time_begin(st);                                                                                 \
       hipLaunchKernelGGL((kern<CI, KT>), dim3(unsigned((ncx + CI - 1) / CI), unsigned(ncy), 1), dim3(CI * KT, 1, 1), \
                          lds, st, a, args...);                                                               \
-      if (t) time_end(st, point_bytes(name) * col_points(name, a));                                          \
+      if (t) time_end(st, point_bytes(name) * col_points(a));                                             \
     }                                                                                                          \
   };
 MI_COL_LAUNCHER(LargePrepL, k_large_prep)
 MI_COL_LAUNCHER(SsColumnL, k_ss_column)
-MI_COL_LAUNCHER(AcousticL, k_acoustic)
+// the extra block rows of a column kernel that runs the spec zone too (ring_blocks), gx blocks of nw >= 4 wavefronts each:
+// at most ny / 2 + 9, so the launch stays within 65535 block rows
+constexpr int kRingRowsMaxNy = 40000;
+int ring_rows(const Args& a, int gx, int nw) {
+  if (a.g.bcx != MI_BC_SPECIFIED || a.g.ny > kRingRowsMaxNy) return 0;
+  const int ncol = 2 * a.g.nx + 2 * (a.g.ny - 2);
+  return ((ncol + nw - 1) / nw + gx - 1) / gx;
+}
+template <int CI, int KT>
+struct AcousticL {
+  static void go(const Args& a, double dts, int it, int ns, hipStream_t st) {
+    const int gx = (a.g.nx + CI - 1) / CI;
+    hipLaunchKernelGGL((k_acoustic<CI, KT>), dim3(unsigned(gx), unsigned(a.g.ny + (KT == 64 ? ring_rows(a, gx, CI * KT / 64) : 0)), 1),
+                       dim3(CI * KT, 1, 1), col_lds_bytes(CI, 10, a.g.nz, 5), st, a, dts, it, ns);
+  }
+};
 MI_COL_LAUNCHER(FinishL, k_finish)
 
 // LDS arrays (per level, extra per column) of each column kernel, in ColKernel order
 constexpr int kColArrays[kNumColKernels][2] = {{1, 0}, {3, 0}, {10, 5}, {1, 1}};
 
 bool col_cfg_fits(int kernel, int cfg, int nz) {
-  if (cfg == kColLevels) return kernel == kColAcoustic;  // the k-march
+  if (cfg == kColLevels) return kernel == kColAcoustic;
   if (cfg < 0 || cfg >= kNumColCfgs) return false;
   if (kernel == kColAcoustic && kColCfgs[cfg][1] < nz + 1) return false;  // one level per thread
   return col_lds_bytes(kColCfgs[cfg][0], kColArrays[kernel][0], nz, kColArrays[kernel][1]) <= kLdsMax;
@@ -4944,7 +4976,8 @@ template <int CI, bool SCAN>
 void levels_go(const Args& a, double dts, int it, int ns, hipStream_t st) {
   // the scans take whole wavefronts: 64 levels, whatever nz
   const int kt = SCAN ? 64 / kAcLpt : (a.g.nz + kAcLpt) / kAcLpt;
-  hipLaunchKernelGGL((k_acoustic_levels<CI, kAcLpt, SCAN>), dim3(unsigned((a.g.nx + CI - 1) / CI), unsigned(a.g.ny), 1),
+  const int gx = (a.g.nx + CI - 1) / CI;
+  hipLaunchKernelGGL((k_acoustic_levels<CI, kAcLpt, SCAN>), dim3(unsigned(gx), unsigned(a.g.ny + (SCAN ? ring_rows(a, gx, CI * kt / 64) : 0)), 1),
                      dim3(unsigned(CI * kt), 1, 1), levels_lds_bytes(CI, kt, kAcLpt, a.g.nz), st, a, dts, it, ns);
 }
 void launch_acoustic_levels(const Args& a, double dts, int it, int ns, hipStream_t st) {
@@ -4954,16 +4987,17 @@ void launch_acoustic_levels(const Args& a, double dts, int it, int ns, hipStream
   else levels_go<2, false>(a, dts, it, ns, st);
 }
 void launch_acoustic(const Args& a, int cfg, double dts, int it, int ns, hipStream_t st) {
+  const int n = a.g.nz + 1;
   // the level kernel's 32-bit byte offsets span one row block (an x-z slice: the whole field)
-  if (cfg == kColLevels && int64_t(a.g.nz + 1) * a.g.sk < (int64_t(1) << 29)) {
-    const bool t = timing("acoustic");
-    if (t) time_begin(st);
-    launch_acoustic_levels(a, dts, it, ns, st);
-    if (t) time_end(st, point_bytes("acoustic") * col_points("acoustic", a));
-  } else {
-    if (cfg == kColLevels) cfg = a.g.nz + 1 <= 64 ? 4 : (a.g.nz + 1 <= 128 ? 5 : 6);
-    dispatch_cfg<AcousticL>(cfg, "acoustic", 10, 5, a.g.nx, a.g.ny, st, a, dts, it, ns);
-  }
+  if (cfg == kColLevels && int64_t(n) * a.g.sk >= (int64_t(1) << 29)) cfg = n <= 64 ? 4 : (n <= 128 ? 5 : 6);
+  const bool t = timing("acoustic");
+  if (t) time_begin(st);
+  if (cfg == kColLevels) launch_acoustic_levels(a, dts, it, ns, st);
+  else dispatch_cfg<AcousticL>(cfg, a, dts, it, ns, st);
+  // the spec zone, where the kernel does not run it
+  const bool own = a.g.ny <= kRingRowsMaxNy && (cfg == kColLevels ? kAcFp32 && n <= 64 : kColCfgs[cfg][1] == 64);
+  if (a.g.spec() && !own) launch_acoustic_ring(a, dts, it, ns, st);
+  if (t) time_end(st, point_bytes("acoustic") * col_points(a));
   launch_open_sums(a, it, ns, st);
 }
 void launch_finish(const Args& a, int cfg, bool prhophi, double hd_dt, hipStream_t st) {
