@@ -86,16 +86,6 @@ inline dim3 grid_of(const Range& r, int by) {
 // registers instead of spilling
 #define MI_POINT_KERNEL __global__ void __launch_bounds__(256)
 
-// the scalar kernels: block z = level + nz * (index in the species list), one species per thread
-#define MI_POINT_INDEX_SP(r)                                           \
-  const Blk blk_ = point_block((r).kfast);                             \
-  const int nk_ = (r).k1 - (r).k0;                                     \
-  const int i = (r).i0 + blk_.x * kBx + int(threadIdx.x);              \
-  const int j = (r).j0 + blk_.y * int(blockDim.y) + int(threadIdx.y);  \
-  const int k = (r).k0 + blk_.z % nk_;                                 \
-  const int sq_ = blk_.z / nk_;                                        \
-  if (i >= (r).i1 || j >= (r).j1) return;
-
 #define MI_POINT_INDEX(r)                          \
   const Blk blk_ = point_block((r).kfast);         \
   const int i = (r).i0 + blk_.x * kBx + int(threadIdx.x); \
@@ -158,19 +148,6 @@ void launch3a(const char* name, double arrays, K kern, Range r, hipStream_t st, 
   const bool t = timing(name);
   if (t) time_begin(st);
   hipLaunchKernelGGL(kern, grid_of(r, by), dim3(kBx, by, 1), 0, st, r, args...);
-  if (t) time_end(st, double(sizeof(real)) * arrays * double(r.i1 - r.i0) * double(r.j1 - r.j0) * double(r.k1 - r.k0));
-}
-// a scalar kernel over the points of r for each of nsp species (grid z = levels x species)
-template <class K, class... T>
-void launch3s(const char* name, double arrays, K kern, Range r, int nsp, hipStream_t st, T... args) {
-  if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0 || nsp <= 0) return;
-  const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
-  r.kfast = point_order();
-  dim3 gr = grid_of(r, by);
-  gr.z *= unsigned(nsp);
-  const bool t = timing(name);
-  if (t) time_begin(st);
-  hipLaunchKernelGGL(kern, gr, dim3(kBx, by, 1), 0, st, r, args...);
   if (t) time_end(st, double(sizeof(real)) * arrays * double(r.i1 - r.i0) * double(r.j1 - r.j0) * double(r.k1 - r.k0));
 }
 template <class K, class... T>
@@ -1675,15 +1652,12 @@ __device__ __forceinline__ double bdiv(double a, double b) {
 // k >= 1 of column (i, j): dampmag sin^2(pi/2 (h_k - h_bot) / zdamp) above h_bot = h_top - zdamp, 0 below, the
 // heights from the stage's saved geopotential.  It does not change within a stage, so the stage's column kernel
 // evaluates it once and the substeps read it.
-__device__ __forceinline__ double damp_weight(const Args& a, int i, int j, int k, double dts) {
-  const Fields& f = a.f;
-  const Geo& g = a.g;
+__device__ __forceinline__ double damp_weight(const Args& a, double htop, real phs, double phb, double dts) {
   const double dampmag = dts * a.q.dampcoef;
   const double hdepth = a.q.zdamp;
   const double pi = 3.141592653589793;  // 4 atan(1), folded
-  const real ph_top = f.ph_save[g.at(i, j, g.nz)], phs = f.ph_save[g.at(i, j, k)];
-  const double htop = bdiv(ph_top + f.phb(i, j, g.nz), kG), hbot = htop - hdepth;
-  const double hk = bdiv(phs + f.phb(i, j, k), kG);
+  const double hbot = htop - hdepth;
+  const double hk = bdiv(phs + phb, kG);
   double dampwt = 0;
   if (hk >= hbot) {
     const double sn = mi_libm::sin(bdiv(H * pi * (hk - hbot), hdepth));
@@ -1761,30 +1735,10 @@ MI_POINT_KERNEL k_ss_prep(Range r, int lv, Args a, int first) {
   }
 }
 
-// p_rho_point (small_step.cpp:97-114): al'' and p'' of one point from phi'' at levels k and k+1;
-// damp: the smdiv divergence damping of the substeps (KWPRho), else the stage start (KPRho)
-__device__ __forceinline__ void p_rho_at(const Args& a, int i, int j, int k, double ph_k, double ph_kp1, double mu2,
-                                         double muts, double t2, bool damp) {
-  const Geo& g = a.g;
-  const Fields& f = a.f;
-  const Lv& c = a.c;
-  const idx_t x = g.at(i, j, k);
-  const double m = c.c1h[k] * muts + c.c2h[k];
-  const double al = -((1. / m) * (f.alt[x] * (c.c1h[k] * mu2) + c.rdnw[k] * (ph_kp1 - ph_k)));
-  put<kHMass>(f.al, g, i, j, k * g.sk, al);
-  double pp = f.c2a[x] * (f.alt[x] * (t2 - c.c1h[k] * mu2 * f.t_save[x]) / (m * (kT0 + f.t_save[x])) - al);
-  if (damp) {
-    const double ptmp = pp;
-    pp = pp + a.q.smdiv * (pp - f.pm1[x]);
-    f.pm1[x] = ptmp;
-  } else {
-    f.pm1[x] = pp;
-  }
-  put<kHMass>(f.p, g, i, j, k * g.sk, pp);
-}
-
 // KPRho (small_step.cpp:116-121) and KCoefW calc_coef_w (small_step.cpp:124-148), dry, one column
-// group: p'', al'' and the b, c, a coefficients in parallel, then the alpha / gamma recurrence
+// group: p'', al'' and the b, c, a coefficients in parallel, then the alpha / gamma recurrence.  A level's loads are issued
+// together and each field read once (c2a was read up to five times); the top geopotential of the damping weight once per
+// column: 271 -> 248 us per launch at 425x300x50 FP32-bulk.  The one-thread recurrence with its division bounds the rest.
 MI_COLUMN_KERNEL k_ss_column(Args a, double cof, double dts) {
   constexpr int kKT = KT;
   extern __shared__ double lds[];
@@ -1802,29 +1756,50 @@ MI_COLUMN_KERNEL k_ss_column(Args a, double cof, double dts) {
     const double m = f.mut[x2];
     const double mu2 = f.mu2[x2], muts = f.muts[x2];
     const double lid = a.q.top_lid ? 0.0 : 1.0;
+    const bool damp = a.q.damp_opt == 3, moist = a.q.moist != 0;
+    const idx_t rj = j * g.sj - kLpad, sk = g.sk;
+    const unsigned eo = unsigned(kLpad + i);
     auto mh = [&](int kk) { return c.c1h[kk] * m + c.c2h[kk]; };
     auto mf = [&](int kk) { return c.c1f[kk] * m + c.c2f[kk]; };
-    auto c2a = [&](int kk) { return f.c2a[g.at(i, j, kk)]; };
-    for (int k = cp.kt; k <= nz; k += kKT) {
-      const idx_t x = g.at(i, j, k);
-      if (k < nz) p_rho_at(a, i, j, k, f.ph2[x], f.ph2[x + g.sk], mu2, muts, f.t2[x], false);
+    const double htop = damp ? bdiv(row_ld(f.ph_save, rj + nz * sk, eo) + f.phb(i, j, nz), kG) : 0.0;
+    for (int k = col_level<CI>(cp.kt); k <= nz; k += kKT) {
+      // a level's loads together, none conditional
+      const idx_t r = rj + k * sk, rm = k > 0 ? r - sk : r, rp = k < nz ? r + sk : r;
+      const real ph_k = row_ld(f.ph2, r, eo), ph_p = row_ld(f.ph2, rp, eo), t2 = row_ld(f.t2, r, eo), ts = row_ld(f.t_save, r, eo);
+      const real alt = row_ld(f.alt, r, eo), c2a = row_ld(f.c2a, r, eo), c2m = row_ld(f.c2a, rm, eo);
+      real cqw = 0, phs = 0;
+      double phb = 0;
+      if (moist) cqw = row_ld(f.cqw, r, eo);
+      if (damp) {
+        phs = row_ld(f.ph_save, r, eo);
+        phb = f.phb(i, j, k);
+      }
+      if (k < nz) {
+        // p_rho_point (small_step.cpp:97-114) at the stage's start: al'' and p''
+        const double mk = c.c1h[k] * muts + c.c2h[k];
+        const double al = -((1. / mk) * (alt * (c.c1h[k] * mu2) + c.rdnw[k] * (double(ph_p) - double(ph_k))));
+        row_st(f.al, r, eo, al);
+        const double pp = c2a * (alt * (double(t2) - c.c1h[k] * mu2 * ts) / (mk * (kT0 + ts)) - al);
+        row_st(f.pm1, r, eo, pp);
+        row_st(f.p, r, eo, pp);
+      }
       // kern::MoistCoef::cq1 = 1 / (1 + cqw), 1 when dry
-      const double cq1 = (a.q.moist && k >= 1 && k < nz) ? 1.0 / (1.0 + f.cqw[x]) : 1.0;
+      const double cq1 = (moist && k >= 1 && k < nz) ? 1.0 / (1.0 + cqw) : 1.0;
       // for the substeps of the stage: cq1 and advance_w's c2a rdnw / (c1h mut + c2h) at the mass levels
-      if (a.q.moist && k >= 1 && k < nz) f.cq1[x] = cq1;
-      if (k < nz) f.cwc[x] = bdiv(double(f.c2a[x]) * c.rdnw[k], c.c1h[k] * m + c.c2h[k]);
+      if (moist && k >= 1 && k < nz) row_st(f.cq1, r, eo, cq1);
+      if (k < nz) row_st(f.cwc, r, eo, bdiv(double(c2a) * c.rdnw[k], c.c1h[k] * m + c.c2h[k]));
       double ak;
       if (k <= 1) ak = 0;
-      else if (k == nz) ak = -2.0 * cof * (c.rdnw[nz - 1] * c.rdnw[nz - 1]) * c2a(nz - 1) * lid / (mh(nz - 1) * mf(nz - 1));
-      else ak = -cq1 * cof * c.rdn[k] * c.rdnw[k - 1] * c2a(k - 1) / (mh(k - 1) * mf(k - 1));
-      f.ca[x] = ak;
+      else if (k == nz) ak = -2.0 * cof * (c.rdnw[nz - 1] * c.rdnw[nz - 1]) * c2m * lid / (mh(nz - 1) * mf(nz - 1));
+      else ak = -cq1 * cof * c.rdn[k] * c.rdnw[k - 1] * c2m / (mh(k - 1) * mf(k - 1));
+      row_st(f.ca, r, eo, ak);
       LDS(AA, k, cp.ci) = ak;
-      if (a.q.damp_opt == 3 && k >= 1) f.dampwt[x] = damp_weight(a, i, j, k, dts);
+      if (damp && k >= 1) row_st(f.dampwt, r, eo, damp_weight(a, htop, phs, phb, dts));
       if (k >= 1 && k < nz) {
-        LDS(B, k, cp.ci) = 1.0 + cq1 * cof * c.rdn[k] * (c.rdnw[k] * c2a(k) / (mh(k) * mf(k)) + c.rdnw[k - 1] * c2a(k - 1) / (mh(k - 1) * mf(k)));
-        LDS(CC, k, cp.ci) = -cq1 * cof * c.rdn[k] * c.rdnw[k] * c2a(k) / (mh(k) * mf(k + 1));
+        LDS(B, k, cp.ci) = 1.0 + cq1 * cof * c.rdn[k] * (c.rdnw[k] * c2a / (mh(k) * mf(k)) + c.rdnw[k - 1] * c2m / (mh(k - 1) * mf(k)));
+        LDS(CC, k, cp.ci) = -cq1 * cof * c.rdn[k] * c.rdnw[k] * c2a / (mh(k) * mf(k + 1));
       } else if (k == nz) {
-        LDS(B, k, cp.ci) = 1.0 + 2.0 * cof * (c.rdnw[nz - 1] * c.rdnw[nz - 1]) * c2a(nz - 1) / (mh(nz - 1) * mf(nz));
+        LDS(B, k, cp.ci) = 1.0 + 2.0 * cof * (c.rdnw[nz - 1] * c.rdnw[nz - 1]) * c2m / (mh(nz - 1) * mf(nz));
       }
     }
   }
@@ -4359,16 +4334,33 @@ MI_POINT_KERNEL k_sc_update(Range r, int lv, Args a, Scalars s, SpList l, double
 
 // rk_update_scalar_pd, first step (KPreUpdatePD, scalars.cpp:174-181): the held tendency folded into
 // q_1 (q_1's halo is refreshed next, as scalars.cpp:383)
-MI_POINT_KERNEL k_sc_pd_pre(Range r, Args a, Scalars s, SpList l, double dt_rk) {
-  MI_POINT_INDEX_SP(r)
+// A level piece per thread, four levels' loads in flight: 194 -> 99 us per launch at 425x300x50 with six species FP32-bulk
+// (one level per thread had two loads behind 300 scalar instructions), 4.6 TB/s.
+MI_POINT_KERNEL k_sc_pd_pre(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
+  const ScPiece pc = sc_piece(r, lv);
+  if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
-  const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
-  const acc m = m_full(a.c, k, f.mub[x2], f.mu1[x2]);
-  {
-    const int n = l.sp[sq_];
-    put<kHMass>(s.q1[n], g, i, j, k * g.sk,
-                qdiv(m * acc(s.q1[n][x]) + acc(dt_rk) * acc((a.q.use_tendf ? s.qtw[n][x] : real(0))), m));
+  const int n = l.sp[pc.sq];
+  const idx_t rj = pc.j * g.sj - kLpad, x2 = g.at2(pc.i, pc.j);
+  const unsigned eo = unsigned(kLpad + pc.i);
+  const double mub = f.mub[x2], mu1 = f.mu1[x2];
+  real* q1 = s.q1[n];
+  const real* qt = a.q.use_tendf ? s.qtw[n] : nullptr;
+  for (int k0 = pc.ka; k0 < pc.kb; k0 += 4) {
+    real q[4], t[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const idx_t row = rj + (k0 + u < pc.kb ? k0 + u : pc.kb - 1) * g.sk;
+      q[u] = row_ld(q1, row, eo);
+      t[u] = qt ? row_ld(qt, row, eo) : real(0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k0 + u < pc.kb) {
+        const acc m = m_full(a.c, k0 + u, mub, mu1);
+        row_st(q1, rj + (k0 + u) * g.sk, eo, qdiv(m * acc(q[u]) + acc(dt_rk) * acc(t[u]), m));
+      }
   }
 }
 
@@ -5119,7 +5111,7 @@ void launch_scalars(const Args& a, const Scalars& s, const int* sp, int n, int s
     case 0: launch_sc_pieces("sc_update", 3 + 4 * n, op, op ? (qv ? k_sc_update<true, true> : k_sc_update<true, false>)
                                                   : (qv ? k_sc_update<false, true> : k_sc_update<false, false>),
                      r, n, st, a, s, l, dt_rk); break;        // q_2 q_1 q_tendf -> q_new
-    case 1: launch3s("sc_pd_pre", 3 * n, k_sc_pd_pre, r, n, st, a, s, l, dt_rk); break;            // q_1 q_tendf -> q_1
+    case 1: launch_sc_pieces("sc_pd_pre", 3 * n, false, k_sc_pd_pre, r, n, st, a, s, l, dt_rk); break;        // q_1 q_tendf -> q_1
     case 2: launch_sc_pieces("sc_pd_scale", 3 + 3 * n, false, k_sc_pd_scale, r, n, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
     default: launch_sc_pieces("sc_pd_update", 3 + 4 * n, op, op ? (qv ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
                                                         : (qv ? k_sc_pd_update<false, true> : k_sc_pd_update<false, false>),
