@@ -4843,10 +4843,7 @@ bool col_cfg_fits(int kernel, int cfg, int nz) {
 }
 
 int col_cfg_default(int kernel, int nx, int ny, int nz) {
-  // the substep kernel: the narrowest one-level-per-thread shape; the others: one level per thread on
-  // small domains (latency); on larger ones 64 columns x 4 levels, a wavefront a row, where the work is the loads and
-  // stores (large_prep, finish: 425x300x50 12.42 -> 12.02 ms a step FP32-bulk, 21.1 -> 20.6 ms FP64, with the kernels'
-  // loads grouped), 16 columns x 16 for the ss column, whose sums over the levels need the narrower block's LDS
+  // the substep kernel: the narrowest one-level-per-thread shape; the others by the number of columns
   if (kernel == kColAcoustic) {
     // FP32-bulk: several levels per thread (425x300x50 557 -> 446 us; FP64 is slower that way, 704 -> 775 us)
     if (kAcFp32) return kColLevels;
@@ -4854,8 +4851,15 @@ int col_cfg_default(int kernel, int nx, int ny, int nz) {
       if (col_cfg_fits(kernel, c, nz)) return c;
     return 6;
   }
-  const bool small = int64_t(nx) * ny <= 16384;
-  const int pref[] = {small ? (nz + 1 <= 64 ? 4 : (nz + 1 <= 128 ? 5 : 6)) : (kernel == kColSsColumn ? 0 : 7), 0, 3, 5, 6};
+  // few columns: one level per thread, for the latency of a column (large_prep, ss_column, finish FP64 at 120x40: 13.9,
+  // 11.9, 8.8 us against 15.0, 15.4, 12.5 with 16 columns x 16).  From 4096 on 16 columns x 16, whose 64-byte rows
+  // waste less of a cache line (large_prep, ss_column, finish FP32-bulk: 64x64x40 20.8, 15.4, 14.8 -> 18.0, 16.9, 14.2 us;
+  // 119x89x44 33.1, 32.5, 24.4 -> 23.9, 23.1, 20.9 us).  On large grids 64 columns x 4, a wavefront a row, where the work
+  // is the loads and stores (large_prep, finish: 425x300x50 187, 232 -> 138, 187 us, but 119x89x44 23.9, 20.9 -> 27.6,
+  // 34.9 us: too few blocks); the ss column's three LDS arrays do not fit that shape.
+  const int64_t cols = int64_t(nx) * ny;
+  const bool small = cols < 4096, large = cols > 16384;
+  const int pref[] = {small ? (nz + 1 <= 64 ? 4 : (nz + 1 <= 128 ? 5 : 6)) : (large && kernel != kColSsColumn ? 7 : 0), 0, 3, 5, 6};
   for (int c : pref)
     if (col_cfg_fits(kernel, c, nz)) return c;
   return 6;
