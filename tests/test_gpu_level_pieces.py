@@ -1,0 +1,52 @@
+"""The kernels that give a thread a run of levels, on grids large enough for runs of several levels (small grids get one
+level per thread), with ragged rows, tiles and last runs; the column kernels' shapes of large grids with them.  FP64: the
+bits of the oracle.  FP32-bulk: within 1e-3 relative L2 of FP64, the bar of its storage (rounding 6e-8 per operation, a
+few hundred operations per step, differences of fields 1e2-1e3 times their result)."""
+import numpy as np
+import pytest
+
+from cppwrf_amd import _abi as A
+from cppwrf_amd.boundary import drifting_boundary
+from cppwrf_amd.dyn import Case, Context, RK3
+from cppwrf_amd.workloads import moist_species, rel_l2
+from oracle_lib import OracleDomain
+
+pytestmark = pytest.mark.gpu
+
+STATE = (A.MI_U, A.MI_V, A.MI_W, A.MI_T, A.MI_PH, A.MI_MU, A.MI_P, A.MI_AL)
+P, S, O, B = A.MI_BC_PERIODIC, A.MI_BC_SYMMETRIC, A.MI_BC_OPEN, A.MI_BC_SPECIFIED
+# runs of 5 levels, of 3, of 2 in a slice; open sides (one level per thread); runs of 3 (the last of 2) and of 5 with the
+# spec zone, the scalars' of 6 (5) and of 4 (2); columns of more than 63 levels with it
+GRIDS = [(198, 149, 45, P, 0), (197, 150, 21, S, 0), (2100, 1, 250, P, 0), (131, 130, 20, O, 0), (201, 143, 23, B, 6), (130, 129, 70, B, 2)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return Context(0)
+
+
+@pytest.mark.parametrize("nx,ny,nz,bc,species", GRIDS)
+def test_runs_of_levels(ctx, nx, ny, nz, bc, species):
+    print(f"[pieces] {nx}x{ny}x{nz} bc {bc} species {species}", flush=True)
+    bdy, extra = None, {}
+    if bc == B:
+        case = Case.hills(nx, ny, nz, dx=15000.0, dt=30.0, seed=9, bc=bc)
+        kw = dict(time_step_sound=4, damp_opt=3, n_moist=species, n_scalars=species, moist_adv_opt=1)
+        bdy, extra = drifting_boundary(case, seed=5), moist_species(case, species, seed=7)
+    else:
+        case = Case.bubble3d(nx, ny, nz, dx=1000.0, ztop=18000.0, dt=2.0, seed=nz, noise_amp=0.3, bc=bc)
+        kw = dict(time_step_sound=4, damp_opt=3, zdamp=5000.0)
+    fields = STATE + tuple(A.MI_Q + n for n in range(species))
+    doms = [RK3(ctx, case.grid, case.params(precision=p, **kw), case) for p in (A.MI_FP64, A.MI_FP32_BULK)]
+    orc = OracleDomain(case, case.params(**kw))
+    for d in doms + [orc]:
+        if bdy:
+            d.load_boundary(bdy)
+        for fid, q in extra.items():
+            d.set_field(fid, q)
+        d.step(2)
+    assert all(d.check_finite() == -1 for d in doms)
+    for fid in fields:
+        assert np.array_equal(doms[0].field(fid).view(np.uint64), orc.field(fid).view(np.uint64)), A.FIELD_NAMES[fid]
+    for fid in (A.MI_U, A.MI_T, A.MI_PH, A.MI_MU):
+        assert rel_l2(doms[1].field(fid), doms[0].field(fid)) <= 1e-3, A.FIELD_NAMES[fid]
