@@ -5,9 +5,9 @@
 // matches is given at each.  Built with -ffp-contract=off: no multiply-add is fused, as the reference.
 // Transcendental calls go to libm_port.hpp, which reproduces the host glibc's pow and sin.
 //
-// Launch shapes: point kernels run one thread per point with 64 consecutive i per wavefront (one
-// 512-byte coalesced row segment per load); column kernels (vertical sums, the tridiagonal solve) run
-// one thread per column and march in k, every load still i-contiguous across the wavefront.
+// Launch shapes: point kernels run one thread per point, or per run of levels of one, with 64 consecutive i
+// per wavefront (one coalesced row segment per load); column kernels (vertical sums, the tridiagonal solve)
+// run several threads per column, a level or a few of them each.
 #include "kernels_fp64.hpp"
 
 #include <cstdlib>
@@ -155,7 +155,8 @@ void launch3(const char* name, K kern, const Range& r, hipStream_t st, T... args
   launch3a(name, point_bytes(name) / double(sizeof(real)), kern, r, st, args...);
 }
 // A level-piece kernel over the points of r: a thread takes lv consecutive levels.  Long pieces share more between
-// levels; short ones keep enough wavefronts (about four per SIMD) on a small grid.
+// levels; short ones keep enough wavefronts (about four per SIMD) on a small grid.  At most 16: with at most 5 a step
+// of 425x300x50 takes the same (11.90 ms), one of 219x173x44 2.31 ms against 2.29.
 int piece_levels(const Range& r, int by, int nsp = 1) {
   const int64_t waves = int64_t(grid_of(r, by).x) * grid_of(r, by).y * by * nsp;  // per level
   const int64_t want = 4096;
@@ -2522,7 +2523,8 @@ MI_COLUMN_KERNEL k_acoustic(Args a, double dts, int it, int ns) {
 // FP32-bulk with two levels per thread takes 161 VGPRs, three wavefronts per SIMD; bounded to four it spills and runs
 // slower (628 us at 425x300x50 with blocks of 16 columns), as four levels per thread (717 us) do.  Blocks of 8 columns
 // (four wavefronts, three blocks per CU) beat 16 and 4 columns.  Substep kernel, FP32-bulk, per launch, against the
-// level-per-thread blocks of 8 x 64: 425x300x50 557 -> 446 us; the step of 219x173x44 3.24 -> 2.65 ms with
+// level-per-thread blocks of 8 x 64: 425x300x50 557 -> 446 us (475 with
+// the spec zone's columns, 29 us in a launch of their own); the step of 219x173x44 3.24 -> 2.65 ms with
 // advance_uv below and without the substeps' halo launches.  In FP64 (197 VGPRs, two wavefronts per SIMD) it is
 // slower (704 -> 775 us), so FP64 keeps the level-per-thread form by default.
 //

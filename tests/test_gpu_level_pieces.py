@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 
 STATE = (A.MI_U, A.MI_V, A.MI_W, A.MI_T, A.MI_PH, A.MI_MU, A.MI_P, A.MI_AL)
 P, S, O, B = A.MI_BC_PERIODIC, A.MI_BC_SYMMETRIC, A.MI_BC_OPEN, A.MI_BC_SPECIFIED
-# runs of 5 levels, of 3, of 2 in a slice; open sides (one level per thread); runs of 3 (the last of 2) and of 5 with the
-# spec zone, the scalars' of 6 (5) and of 4 (2); columns of more than 63 levels with it
+# runs of 6 levels (the last of 3), of 3, of 2 in a slice; open sides (one level per thread); runs of 3 (2) and of 6 (4)
+# with the spec zone, the scalars' of 12; columns of more than 63 levels with it
 GRIDS = [(198, 149, 45, P, 0), (197, 150, 21, S, 0), (2100, 1, 250, P, 0), (131, 130, 20, O, 0), (201, 143, 23, B, 6), (130, 129, 70, B, 2)]
 
 
