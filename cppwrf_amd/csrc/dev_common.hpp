@@ -64,6 +64,27 @@ struct BField {
   __device__ double operator()(int i, int j, int k) const { return p[i * si + j * sj + k * sk]; }
 };
 
+// A wavefront's view of a field: 64 consecutive points of one row (j and k are the same for all its lanes), so an
+// access is a scalar row address + the lane's 32-bit offset from the row's start (8 points west of i = 0).  Only a
+// point's place in its row goes into the 32-bit offset: an x-z slice's levels can span more than 2^32 bytes.
+template <class T>
+__host__ __device__ __forceinline__ T row_ld(const T* p, idx_t row, unsigned eo) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
+}
+template <class T>
+__host__ __device__ __forceinline__ void row_st(T* p, idx_t row, unsigned eo, double v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(p + row) + eo * unsigned(sizeof(T))) = T(v);
+}
+// The levels of a base-state field at one point of the row that starts at index row: the full field's, or the profile's
+struct BaseLevels {
+  const double* p;
+  idx_t row, sk;
+  unsigned eo;
+  __host__ __device__ BaseLevels(const BField& b, idx_t row_, unsigned eo_)
+      : p(b.p), row(b.si ? row_ : 0), sk(b.sk), eo(b.si ? eo_ : 0u) {}
+  __host__ __device__ double operator()(int k) const { return row_ld(p, row + k * sk, eo); }
+};
+
 // vertical coefficients (device copies of the level arrays)
 struct Lv {
   const double *dnw, *rdnw, *dn, *rdn, *fnm, *fnp, *c1h, *c2h, *c3h, *c4h, *c1f, *c2f, *c3f, *c4f;

@@ -397,17 +397,6 @@ constexpr int kChain = 8;
 #define LDS(arr, k, ci) (arr)[(k) * CI + (ci)]
 
 // ----------------------------------------------------------------------------- level pieces
-// A wavefront's view of the fields: 64 consecutive points of one row (j and k are the same for all its lanes), so an
-// access is a scalar row address + the lane's 32-bit offset from the row's start (8 points west of i = 0).
-template <class T>
-__device__ __forceinline__ T row_ld(const T* p, idx_t row, unsigned eo) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p + row) + eo * unsigned(sizeof(T)));
-}
-template <class T>
-__device__ __forceinline__ void row_st(T* p, idx_t row, unsigned eo, double v) {
-  *reinterpret_cast<T*>(reinterpret_cast<char*>(p + row) + eo * unsigned(sizeof(T))) = T(v);
-}
-
 // A block of the level-piece kernels: 64 points of four rows (a wavefront per row) x lv levels; the block grid is
 // x tiles, y tiles, level pieces, dealt to the XCDs in eighths, the pieces of a tile back to back (point_block)
 struct Piece {
@@ -695,8 +684,7 @@ __device__ __forceinline__ void tend_uv_levels(const Args& a, int i, int j, int 
   double dn;
   if (ka == 0) dn = H * (c.cf1 * psum(0) + c.cf2 * psum(1) + c.cf3 * psum(2));
   else dn = H * (c.fnm[ka] * (pb_ + p0) + c.fnp[ka] * psum(ka - 1));
-  const idx_t pbj = f.pb.si ? rj : 0, pbb = f.pb.si ? rb : 0;
-  const unsigned pbo = f.pb.si ? at.eo : 0u, pbw = f.pb.si ? at.eo + unsigned(db) : 0u;
+  const BaseLevels pb(f.pb, rj, at.eo), pbx(f.pb, rb, at.eo + unsigned(db));  // at the point, across the face
   for (int k = ka; k < kb; ++k) {
     const idx_t r0 = rj + k * sk, r1 = rb + k * sk, rsk = rs + k * sk;
     const real* qx = at(w, r0);
@@ -718,8 +706,7 @@ __device__ __forceinline__ void tend_uv_levels(const Args& a, int i, int j, int 
     const real rw0p = at(f.rw, r0 + sk)[0], rwbp = at(f.rw, r1 + sk)[db];
     const real at0 = at(f.alt, r0)[0], atb = at(f.alt, r1)[db], al0 = at(f.al, r0)[0], alb_ = at(f.al, r1)[db];
     const double fp0 = at(f.php, r0)[0], fpb = at(f.php, r1)[db];
-    const unsigned bk = unsigned(k) * unsigned(f.pb.sk);
-    const double pbv = row_ld(f.pb.p, pbj, pbo + bk), pbvb = row_ld(f.pb.p, pbb, pbw + bk);
+    const double pbv = pb(k), pbvb = pbx(k);
     const real cqk = at(moist ? cq : f.alt, r0)[0], hk = at(a.q.use_tendf ? held : f.alt, r0)[0];
     // the cross wind of the curvature term: v at (i - 1, i) x (j, j + 1) for u, u at (i, i + 1) x (j - 1, j) for v
     const real* cw = DIR == 0 ? f.v2 : f.u2;
@@ -1890,8 +1877,7 @@ __device__ __forceinline__ void uv_levels(const Args& a, int i, int j, int ka, i
   }
   hu = F(rmu * c.rdx);
   hv = F(rmv * c.rdy);
-  const idx_t pbj = f.pb.si ? rj : 0, pbs = f.pb.si ? rs : 0;  // the base pressure: a full field, or a profile
-  const unsigned pbo = f.pb.si ? eo : 0u, pbw = f.pb.si ? ew : 0u;
+  const BaseLevels pb(f.pb, rj, eo), pbw(f.pb, rj, ew), pbs(f.pb, rs, eo);  // at the point, west and south of it
   // the pressure sum across a face at level m, and its average onto w level kk (FP64: large_step's expressions)
   auto psum = [&](int m, bool v) -> F {
     return F(row_ld(f.p, rj + m * sk, eo)) + F(v ? row_ld(f.p, rs + m * sk, eo) : row_ld(f.p, rj + m * sk, ew));
@@ -1923,8 +1909,7 @@ __device__ __forceinline__ void uv_levels(const Args& a, int i, int j, int ka, i
     const real h0p = row_ld(f.ph2, r0 + sk, eo), hwp = row_ld(f.ph2, r0 + sk, ew), hsp = row_ld(f.ph2, r1 + sk, eo);
     const real p0p = row_ld(f.p, r0 + sk, eo), pwp = row_ld(f.p, r0 + sk, ew), psp = row_ld(f.p, r1 + sk, eo);
     const real qu = row_ld(moist ? f.cqu : f.u2, r0, eo), qv = row_ld(moist ? f.cqv : f.v2, r0, eo);
-    const unsigned bk = unsigned(k) * unsigned(f.pb.sk);
-    const double pb0 = row_ld(f.pb.p, pbj, pbo + bk), pbwv = row_ld(f.pb.p, pbj, pbw + bk), pbsv = row_ld(f.pb.p, pbs, pbo + bk);
+    const double pb0 = pb(k), pbwv = pbw(k), pbsv = pbs(k);
     const double c1 = c.c1h[k], c2 = c.c2h[k], rdnw = c.rdnw[k];
     F upu, upv;  // the averaged pressure sums at w level k + 1
     if (k + 1 == nz) {
