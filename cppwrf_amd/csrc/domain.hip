@@ -1374,6 +1374,7 @@ void fused_prepare(mi_domain* const* ms, int n, void* dev, hipStream_t st, Fused
     as[size_t(q)] = &d->a;
     info.nzmax = std::max(info.nzmax, d->grid.nz);
   }
+  info.levels = batch_levels(as.data(), n);
   std::vector<BatchMember> tabs(6 * size_t(n + 1));
   for (int rk = 1; rk <= 3; ++rk) {
     std::vector<double> dts(static_cast<size_t>(n));
@@ -1423,8 +1424,8 @@ void fused_capture(mi_domain* const* ms, int n, hipStream_t s0, const hipStream_
       });
       for (int it = 1; it <= ns; ++it) {
         launch_uv_batch(dev_args, tabs + size_t(rk - 1) * size_t(n + 1), n, info.blocks_uv[rk - 1], s0);
-        launch_acoustic_batch(dev_args, tabs + size_t(rk + 2) * size_t(n + 1), n, info.blocks_ac[rk - 1], info.nzmax, it, ns,
-                              s0);
+        launch_acoustic_batch(dev_args, tabs + size_t(rk + 2) * size_t(n + 1), n, info.blocks_ac[rk - 1], info.nzmax,
+                              info.levels, it, ns, s0);
         branch([rk, it](Domain& m) {
           launch_open_sums(m.a, it, m.stage_ns(rk), m.stream());
           m.after_acoustic(rk, it);

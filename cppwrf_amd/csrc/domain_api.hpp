@@ -70,9 +70,11 @@ struct mi_domain {
   virtual bool fusable() const = 0;
 };
 
-// what a fused batch step launches with: the acoustic step count, the largest nz, each stage's block counts
+// what a fused batch step launches with: the acoustic step count, the largest nz, the form of the substep kernel
+// (several levels per thread), each stage's block counts
 struct FusedInfo {
   int ns = 0, nzmax = 0;
+  bool levels = false;
   int blocks_uv[3] = {0, 0, 0}, blocks_ac[3] = {0, 0, 0};
 };
 

@@ -2966,8 +2966,9 @@ MI_POINT_KERNEL k_uv_batch(const Args* as, const BatchMember* tab, int n) {
   if (i >= t.i1 || j >= t.j1) return;
   uv_levels<true>(as[m], i, j, k, k + kBatchLv < t.k1 ? k + kBatchLv : t.k1, t.dts);  // the open-boundary forms are taken only where a member's grid is open
 }
-// the substep's column kernel of every member (blocks of CI columns x KT levels; KT >= nz + 1 of every member)
-template <int CI, int KT>
+// the substep's column kernel of every member (blocks of CI columns x KT levels; KT >= nz + 1 of every member); LEVELS:
+// kAcLpt levels per thread (batch_levels), the same bits
+template <int CI, int KT, bool LEVELS>
 __global__ void __launch_bounds__(CI * KT) k_acoustic_batch(const Args* as, const BatchMember* tab, int n, int it, int ns) {
   extern __shared__ double lds[];
   const Blk b = xcd_block();
@@ -2979,7 +2980,7 @@ __global__ void __launch_bounds__(CI * KT) k_acoustic_batch(const Args* as, cons
   cp.kt = int(threadIdx.x) / CI;
   cp.i = (l % t.gx) * CI + cp.ci;
   cp.j = l / t.gx;
-  if constexpr (kAcFp32) acoustic_levels<CI, kAcLpt, true>(as[m], l % t.gx, l / t.gx, lds, t.dts, it, ns);  // the bits it gives alone
+  if constexpr (LEVELS) acoustic_levels<CI, kAcLpt, true>(as[m], l % t.gx, l / t.gx, lds, t.dts, it, ns);
   else acoustic_cols<CI, KT>(as[m], cp, lds, t.dts, it, ns);
 }
 
@@ -4937,16 +4938,27 @@ int batch_table_acoustic(const Args* const* as, const double* dts, int n, BatchM
   return start;
 }
 bool batch_fits(const Args& a) { return a.g.nz + 1 <= kBatchKT; }
+// The form with several levels per thread reaches a row block (an x-z slice: the whole field) with 32-bit byte offsets
+bool levels_span(const Args& a) { return int64_t(a.g.nz + 1) * a.g.sk < (int64_t(1) << 29); }
+int acoustic_cfg(const Args& a, int cfg) {
+  if (cfg != kColLevels || levels_span(a)) return cfg;
+  return a.g.nz + 1 <= 64 ? 4 : (a.g.nz + 1 <= 128 ? 5 : 6);
+}
+bool batch_levels(const Args* const* as, int n) {
+  for (int m = 0; m < n; ++m)
+    if (!levels_span(*as[m])) return false;
+  return kAcFp32;
+}
 void launch_uv_batch(const Args* dev_args, const BatchMember* dev_tab, int n, int blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_uv_batch, dim3(unsigned(blocks), 1, 1), dim3(kBx, 4, 1), 0, st, dev_args, dev_tab, n);
 }
-void launch_acoustic_batch(const Args* dev_args, const BatchMember* dev_tab, int n, int blocks, int nzmax, int it, int ns,
-                           hipStream_t st) {
-  const int kt = kAcFp32 ? 64 / kAcLpt : kBatchKT;
-  const size_t lds = kAcFp32 ? levels_lds_bytes(kBatchCI, kt, kAcLpt, nzmax)
-                             : col_lds_bytes(kBatchCI, kColArrays[kColAcoustic][0], nzmax, kColArrays[kColAcoustic][1]);
-  hipLaunchKernelGGL((k_acoustic_batch<kBatchCI, kBatchKT>), dim3(unsigned(blocks), 1, 1), dim3(unsigned(kBatchCI * kt), 1, 1),
-                     lds, st, dev_args, dev_tab, n, it, ns);
+void launch_acoustic_batch(const Args* dev_args, const BatchMember* dev_tab, int n, int blocks, int nzmax, bool levels,
+                           int it, int ns, hipStream_t st) {
+  const int kt = levels ? 64 / kAcLpt : kBatchKT;
+  const size_t lds = levels ? levels_lds_bytes(kBatchCI, kt, kAcLpt, nzmax)
+                            : col_lds_bytes(kBatchCI, kColArrays[kColAcoustic][0], nzmax, kColArrays[kColAcoustic][1]);
+  hipLaunchKernelGGL((levels ? k_acoustic_batch<kBatchCI, kBatchKT, kAcFp32> : k_acoustic_batch<kBatchCI, kBatchKT, false>),
+                     dim3(unsigned(blocks), 1, 1), dim3(unsigned(kBatchCI * kt), 1, 1), lds, st, dev_args, dev_tab, n, it, ns);
 }
 // KSumEdge of the open directions after a substep's column kernel
 void launch_open_sums(const Args& a, int it, int ns, hipStream_t st) {
@@ -4971,8 +4983,7 @@ void launch_acoustic_levels(const Args& a, double dts, int it, int ns, hipStream
 }
 void launch_acoustic(const Args& a, int cfg, double dts, int it, int ns, hipStream_t st) {
   const int n = a.g.nz + 1;
-  // the level kernel's 32-bit byte offsets span one row block (an x-z slice: the whole field)
-  if (cfg == kColLevels && int64_t(n) * a.g.sk >= (int64_t(1) << 29)) cfg = n <= 64 ? 4 : (n <= 128 ? 5 : 6);
+  cfg = acoustic_cfg(a, cfg);
   const bool t = timing("acoustic");
   if (t) time_begin(st);
   if (cfg == kColLevels) launch_acoustic_levels(a, dts, it, ns, st);

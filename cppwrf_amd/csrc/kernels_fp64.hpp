@@ -204,9 +204,13 @@ constexpr int kMaxBatch = 64;
 int batch_table_uv(const Args* const* as, const double* dts, int n, BatchMember* out);
 int batch_table_acoustic(const Args* const* as, const double* dts, int n, BatchMember* out);
 bool batch_fits(const Args& a);  // the batched column kernel's levels per block hold the member's
+// the substep kernel's shape for a domain tuned to cfg, and whether a batch's takes several levels per thread: not
+// where that form's offsets do not span a member
+int acoustic_cfg(const Args& a, int cfg);
+bool batch_levels(const Args* const* as, int n);
 void launch_uv_batch(const Args* dev_args, const BatchMember* dev_tab, int n, int blocks, hipStream_t st);
-void launch_acoustic_batch(const Args* dev_args, const BatchMember* dev_tab, int n, int blocks, int nzmax, int it, int ns,
-                           hipStream_t st);
+void launch_acoustic_batch(const Args* dev_args, const BatchMember* dev_tab, int n, int blocks, int nzmax, bool levels,
+                           int it, int ns, hipStream_t st);
 void launch_finish(const Args& a, int cfg, bool prhophi, double hd_dt, hipStream_t st);
 // the held tendencies of u, v, w, theta at the first stage: kSixthZero zeroes them and adds the sixth-order
 // diffusion; kSixthKeep adds it to what they hold (a physics plugin's part2); kSixthZeroOnly only zeroes
