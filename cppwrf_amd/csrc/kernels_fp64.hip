@@ -10,6 +10,7 @@
 // run several threads per column, a level or a few of them each.
 #include "kernels_fp64.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -1341,17 +1342,20 @@ MI_POINT_KERNEL k_tend_w(Range r, int lv, Args a) {
 // KTendT (large_step.cpp:502-565)
 template <bool OPEN, bool THF>
 MI_POINT_KERNEL k_tend_t(Range r, int lv, Args a) {
-  const Piece pc = level_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  // Open sides and the plugin's forcing, whose terms the march does not form: a level per thread (with RTHFTEN a step's
+  // three launches at 425x300x50 took 555 us FP32-bulk, 807 FP64 as a loop over a run's levels, 377 and 620 so)
+  constexpr bool kOne = OPEN || THF;
+  const Piece pc = level_piece(r, kOne ? 1 : lv);
   if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
   const Lv& c = a.c;
   const int i = pc.i, j = pc.j;
-  if (!OPEN && !(THF && f.thf) && tend_inner<false>(g, j)) {
+  if (!kOne && tend_inner<false>(g, j)) {
     tend_t_levels(a, i, j, pc.ka, pc.kb);
     return;
   }
-  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
+  for (int k = pc.ka; k < (kOne ? pc.ka + 1 : pc.kb); ++k) {
   const int nz = g.nz;
   const idx_t sj = g.sj, sk = g.sk;
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j);
@@ -4269,7 +4273,8 @@ __device__ __forceinline__ ScPiece sc_piece(const Range& r, int lv) {
 // every species of the list; the new values go to the species' second buffer
 template <bool OPEN, bool QVF>
 MI_POINT_KERNEL k_sc_update(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
-  const ScPiece pc = sc_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  constexpr bool kOne = OPEN || QVF;  // open sides, RQVFTEN: a level per thread
+  const ScPiece pc = sc_piece(r, kOne ? 1 : lv);
   if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
@@ -4277,12 +4282,12 @@ MI_POINT_KERNEL k_sc_update(Range r, int lv, Args a, Scalars s, SpList l, double
   const int i = pc.i, j = pc.j, sq_ = pc.sq;
   {
     const int n = l.sp[sq_];
-    if (!OPEN && !(QVF && f.qvf && n == 0) && sc_inner(g, j)) {
+    if (!kOne && sc_inner(g, j)) {
       sc_levels<0>(a, s.q2[n], s.q1[n], nullptr, a.q.use_tendf ? s.qtw[n] : nullptr, s.qn[n], i, j, pc.ka, pc.kb, acc(dt_rk));
       return;
     }
   }
-  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
+  for (int k = pc.ka; k < (kOne ? pc.ka + 1 : pc.kb); ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j), x0 = g.at(i, j, 0);
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc m_old = m_full(c, k, f.mub[x2], f.mu1[x2]), m_new = m_full(c, k, f.mub[x2], f.mu2[x2]);
@@ -4427,7 +4432,8 @@ MI_POINT_KERNEL k_sc_pd_scale(Range r, int lv, Args a, Scalars s, SpList l, doub
 // advect_scalar_pd's limited divergence and rk_update_scalar (KUpdatePD, scalars.cpp:252-291)
 template <bool OPEN, bool QVF>
 MI_POINT_KERNEL k_sc_pd_update(Range r, int lv, Args a, Scalars s, SpList l, double dt_rk) {
-  const ScPiece pc = sc_piece(r, OPEN ? 1 : lv);  // open sides: a level per thread
+  constexpr bool kOne = OPEN || QVF;  // open sides, RQVFTEN: a level per thread
+  const ScPiece pc = sc_piece(r, kOne ? 1 : lv);
   if (!pc.on) return;
   const Geo& g = a.g;
   const Fields& f = a.f;
@@ -4436,12 +4442,12 @@ MI_POINT_KERNEL k_sc_pd_update(Range r, int lv, Args a, Scalars s, SpList l, dou
   const int i = pc.i, j = pc.j, sq_ = pc.sq;
   {
     const int n = l.sp[sq_];
-    if (!OPEN && !(QVF && f.qvf && n == 0) && sc_inner(g, j)) {
+    if (!kOne && sc_inner(g, j)) {
       sc_levels<2>(a, s.q2[n], s.q1[n], s.scale[n], nullptr, s.qn[n], i, j, pc.ka, pc.kb, acc(dt_rk));
       return;
     }
   }
-  for (int k = pc.ka; k < (OPEN ? pc.ka + 1 : pc.kb); ++k) {
+  for (int k = pc.ka; k < (kOne ? pc.ka + 1 : pc.kb); ++k) {
   const idx_t x = g.at(i, j, k), x2 = g.at2(i, j), sj = g.sj, sk = g.sk;
   const acc msftx = acc(f.msftx[x2]), msfty = acc(f.msfty[x2]);
   const acc m_old = m_full(c, k, f.mub[x2], f.mu1[x2]), m_new = m_full(c, k, f.mub[x2], f.mu2[x2]);
@@ -4866,8 +4872,8 @@ void launch_tendencies(const Args& a, hipStream_t st) {
   const bool op = g.ox() || g.oy();
   // Level marches; with open sides, whose edge columns take their own terms, a level per thread (97x75x35 FP64, where
   // every wavefront holds an open column: the step 0.89 ms that way, 0.96 with the march's code around it)
-  auto go = [&](const char* name, auto kern, const Range& r) {
-    if (op) launch_level(name, kern, r, st, a);
+  auto go = [&](const char* name, auto kern, const Range& r, bool one = false) {
+    if (op || one) launch_level(name, kern, r, st, a);
     else launch_pieces(name, point_bytes(name), kern, r, st, a);
   };
   go("tend_u", op ? k_tend_u<true> : k_tend_u<false>, Range{g.ox() ? 0 : ui0, g.ox() ? g.nx + 1 : g.nx, 0, g.ny, 0, g.nz});
@@ -4876,7 +4882,7 @@ void launch_tendencies(const Args& a, hipStream_t st) {
   go("tend_w", op ? k_tend_w<true> : k_tend_w<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1});
   go("tend_t", op ? (a.f.thf ? k_tend_t<true, true> : k_tend_t<true, false>)
                   : (a.f.thf ? k_tend_t<false, true> : k_tend_t<false, false>),
-     Range{0, g.nx, 0, g.ny, 0, g.nz});
+     Range{0, g.nx, 0, g.ny, 0, g.nz}, a.f.thf != nullptr);
   go("tend_ph", op ? k_tend_ph<true> : k_tend_ph<false>, Range{0, g.nx, 0, g.ny, 1, g.nz + 1});
 }
 
@@ -5102,23 +5108,38 @@ void launch_pd_geom(const Args& a, double dt, hipStream_t st) {
 
 void launch_scalars(const Args& a, const Scalars& s, const int* sp, int n, int step, double dt_rk, hipStream_t st) {
   if (n <= 0) return;
-  SpList l{};
-  l.n = n;
-  for (int q = 0; q < n; ++q) l.sp[q] = sp[q];
   const Geo& g = a.g;
   const Range r{0, g.nx, 0, g.ny, 0, g.nz};
   // the open-boundary terms and the RQVFTEN store compiled in only where used
-  const bool op = g.ox() || g.oy(), qv = a.f.qvf != nullptr;
-  switch (step) {
-    case 0: launch_sc_pieces("sc_update", 3 + 4 * n, op, op ? (qv ? k_sc_update<true, true> : k_sc_update<true, false>)
-                                                  : (qv ? k_sc_update<false, true> : k_sc_update<false, false>),
-                     r, n, st, a, s, l, dt_rk); break;        // q_2 q_1 q_tendf -> q_new
-    case 1: launch_sc_pieces("sc_pd_pre", 3 * n, false, k_sc_pd_pre, r, n, st, a, s, l, dt_rk); break;        // q_1 q_tendf -> q_1
-    case 2: launch_sc_pieces("sc_pd_scale", 3 + 3 * n, false, k_sc_pd_scale, r, n, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
-    default: launch_sc_pieces("sc_pd_update", 3 + 4 * n, op, op ? (qv ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
-                                                        : (qv ? k_sc_pd_update<false, true> : k_sc_pd_update<false, false>),
-                      r, n, st, a, s, l, dt_rk); break; // q_2 q_1 scale -> q_new
+  const bool op = g.ox() || g.oy(), qv = a.f.qvf != nullptr && (step == 0 || step == 3);
+  // RQVFTEN is the vapour's: species 0 alone takes the level-per-thread form that stores it, the others march (six
+  // species, rk_update_scalar of a step with the vapour a loop over a run's levels: 119x89x44 131 us FP32-bulk, 239 FP64;
+  // so 104 and 183; 425x300x50 757 and 1637, so 769 and 1515)
+  int rest[MI_MAX_SCALARS], nrest = 0;
+  if (qv && !op && n > 1) {
+    for (int q = 0; q < n; ++q)
+      if (sp[q] != 0) rest[nrest++] = sp[q];
   }
+  SpList l{};
+  auto go = [&](const int* list, int m, bool f) {
+    l.n = m;
+    for (int q = 0; q < m; ++q) l.sp[q] = list[q];
+    switch (step) {
+      case 0: launch_sc_pieces("sc_update", 3 + 4 * m, op || f, op ? (f ? k_sc_update<true, true> : k_sc_update<true, false>)
+                                                                : (f ? k_sc_update<false, true> : k_sc_update<false, false>),
+                               r, m, st, a, s, l, dt_rk); break;        // q_2 q_1 q_tendf -> q_new
+      case 1: launch_sc_pieces("sc_pd_pre", 3 * m, false, k_sc_pd_pre, r, m, st, a, s, l, dt_rk); break;        // q_1 q_tendf -> q_1
+      case 2: launch_sc_pieces("sc_pd_scale", 3 + 3 * m, false, k_sc_pd_scale, r, m, st, a, s, l, dt_rk); break;    // q_2 q_1 -> scale
+      default: launch_sc_pieces("sc_pd_update", 3 + 4 * m, op || f, op ? (f ? k_sc_pd_update<true, true> : k_sc_pd_update<true, false>)
+                                                                      : (f ? k_sc_pd_update<false, true> : k_sc_pd_update<false, false>),
+                                r, m, st, a, s, l, dt_rk); break; // q_2 q_1 scale -> q_new
+    }
+  };
+  const bool vapour = qv && std::find(sp, sp + n, 0) != sp + n;
+  if (nrest == 0 || nrest == n) return go(sp, n, vapour);
+  const int first = 0;
+  go(&first, 1, true);
+  go(rest, nrest, false);
 }
 void launch_bdy(const Args& a, const Scalars& s, const BdySet& bs, BdyMode mode, hipStream_t st) {
   if (bs.n <= 0) return;

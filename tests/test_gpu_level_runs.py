@@ -1,0 +1,71 @@
+"""Options and boundaries with runs of several levels per thread (grids with enough wavefronts per level), two steps.
+
+FP64: every prognostic field, species and forcing has the oracle's bits.
+
+FP32-bulk: the change of every field over the two steps is within 5 % (relative L2) of FP64's.  Storage rounds a value
+by 6e-8 of it about ten times in two steps; the fields change by 1e-5 of their size or more in them, so rounding makes
+up to 2 % of the change, while a flux missing or misplaced at the seams of runs of 2 to 6 levels makes tens of per
+cent."""
+import numpy as np
+import pytest
+
+from conftest import bitwise_equal, first_diff
+from cppwrf_amd import _abi as A
+from cppwrf_amd.boundary import drifting_boundary
+from cppwrf_amd.dyn import Case, Context, RK3
+from cppwrf_amd.workloads import moist_species, rel_l2
+from oracle_lib import OracleDomain
+from physics_plugin import Plugin
+
+pytestmark = pytest.mark.gpu
+
+STATE = (A.MI_U, A.MI_V, A.MI_W, A.MI_T, A.MI_PH, A.MI_MU, A.MI_P, A.MI_AL)
+P, O, B = A.MI_BC_PERIODIC, A.MI_BC_OPEN, A.MI_BC_SPECIFIED
+
+
+def _hills(bc, seed, nz=20):
+    return lambda: Case.hills(198, 121, nz, dx=15000.0, dt=60.0, seed=seed, bc=bc)
+
+
+CASES = {  # name: (case, parameters, the plugin's forcings kept)
+    # the vapour stores RQVFTEN, level by level, beside species whose runs march: plain and limited, in one list or two
+    "forcing_periodic": (_hills(P, 3), dict(n_moist=2, n_scalars=4, moist_adv_opt=1, scalar_adv_opt=0), True),
+    "forcing_specified": (_hills(B, 4), dict(n_moist=3, n_scalars=3, moist_adv_opt=1), True),
+    "forcing_plain": (_hills(P, 5), dict(n_moist=1, n_scalars=1, moist_adv_opt=0), True),
+    "forcing_tracer_limited": (_hills(P, 6), dict(n_moist=1, n_scalars=2, moist_adv_opt=0, scalar_adv_opt=1), True),
+}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return Context(0)
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_runs_of_levels(ctx, name):
+    print(f"[level runs] {name}", flush=True)
+    make, opts, forcing = CASES[name]
+    case = make()
+    kw = dict(dict(time_step_sound=4, damp_opt=3, zdamp=5000.0), **opts)
+    ns = kw.get("n_scalars", 0)
+    doms = [RK3(ctx, case.grid, case.params(precision=p, **kw), case) for p in (A.MI_FP64, A.MI_FP32_BULK)]
+    orc = OracleDomain(case, case.params(**kw))
+    fids = STATE + tuple(A.MI_Q + n for n in range(ns))
+    for d in doms + [orc]:
+        if case.grid.bc_x == B:
+            d.load_boundary(drifting_boundary(case, seed=5))
+        for fid, q in (moist_species(case, ns, seed=7) if ns else {}).items():
+            d.set_field(fid, q)
+        if forcing:
+            d.set_column_physics(Plugin(True, True, ns))
+    before = [{f: d.field(f) for f in fids} for d in doms]
+    for d in doms + [orc]:
+        d.step(2)
+    for fid in fids + ((A.MI_TH_FORCING, A.MI_QV_FORCING) if forcing else ()):
+        a, b = doms[0].field(fid), orc.field(fid)
+        assert bitwise_equal(a, b), f"{A.FIELD_NAMES[fid]}: {first_diff(a, b)}"
+    for fid in fids:
+        change = [d.field(fid) - b[fid] for d, b in zip(doms, before)]
+        e = rel_l2(change[1], change[0])
+        print(f"[level runs] {name} {A.FIELD_NAMES[fid]}: {e:.2e}", flush=True)
+        assert e <= 5e-2, A.FIELD_NAMES[fid]
