@@ -314,13 +314,10 @@ struct Domain final : mi_domain {
     // the microphysics heating leaves theta_m at the last stage with moisture (small_step.cpp:602)
     const double hd_dt = (rk == 3 && a.q.moist) ? dts * double(ns) : 0.0;
     launch_finish(a, colcfg[kColFinish], prhophi, hd_dt, st);
-    // small_step.cpp:606 (and 616: p, al of the fused calc_p_rho_phi)
-    if (prhophi)
-      halo({{f.u2, -1, -1}, {f.v2, -1, -1}, {f.w2, -1, -1}, {f.t2, -1, -1}, {f.ph2, -1, -1}, {f.ww, -1, -1},
-            {f.mu2, -1, -1}, {f.p, -1, -1}, {f.al, -1, -1}});
-    else
-      halo({{f.u2, -1, -1}, {f.v2, -1, -1}, {f.w2, -1, -1}, {f.t2, -1, -1}, {f.ph2, -1, -1}, {f.ww, -1, -1},
-            {f.mu2, -1, -1}});
+    // small_step.cpp:606, and p, al: of the fused calc_p_rho_phi (:616), or p'', al'' of the last substep (:593), which a
+    // caller who steps phase by phase sees through the fields' views
+    halo({{f.u2, -1, -1}, {f.v2, -1, -1}, {f.w2, -1, -1}, {f.t2, -1, -1}, {f.ph2, -1, -1}, {f.ww, -1, -1},
+          {f.mu2, -1, -1}, {f.p, -1, -1}, {f.al, -1, -1}});
   }
 
   // ScalarTransport::run_stage (scalars.cpp:436-461): the plain species, then the positive-definite ones
