@@ -51,7 +51,7 @@ __device__ __forceinline__ Blk xcd_block() {
 
 struct Range {
   int i0, i1, j0, j1, k0, k1;
-  int kfast;  // the block order of a point kernel (below)
+  int kfast = 0;  // the block order of a point kernel (below)
 };
 
 // The point kernels' blocks (64 i x 4 j at one level) in level-fastest order: the n-th block of an XCD's share is
@@ -70,7 +70,7 @@ __device__ __forceinline__ Blk point_block(int kfast) {
   b.y = int(l / (gz * gx));
   return b;
 }
-// the order point kernels launch with: level-fastest unless MI_BLOCK_ORDER=ijk (for timing the two)
+// the order point kernels, level pieces included, launch with: level-fastest unless MI_BLOCK_ORDER=ijk (for timing the two)
 int point_order() {
   static const int o = [] {
     const char* e = std::getenv("MI_BLOCK_ORDER");
@@ -173,6 +173,7 @@ void launch_sc_pieces(const char* name, double arrays, bool one_level, K kern, R
   if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0 || nsp <= 0) return;
   const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
   const int lv = one_level ? 1 : piece_levels(r, by, nsp);
+  r.kfast = point_order();
   dim3 gr = grid_of(r, by);
   gr.z = unsigned((r.k1 - r.k0 + lv - 1) / lv) * unsigned(nsp);
   const bool t = timing(name);
@@ -184,7 +185,7 @@ template <class K, class... T>
 void launch_pieces(const char* name, double bytes, K kern, Range r, hipStream_t st, T... args) {
   if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0) return;
   const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
-  r.kfast = 1;
+  r.kfast = point_order();
   const int lv = piece_levels(r, by);
   dim3 gr = grid_of(r, by);
   gr.z = unsigned((r.k1 - r.k0 + lv - 1) / lv);
@@ -198,6 +199,7 @@ template <class K, class... T>
 void launch_level(const char* name, K kern, Range r, hipStream_t st, T... args) {
   if (r.i1 <= r.i0 || r.j1 <= r.j0 || r.k1 <= r.k0) return;
   const int by = (r.j1 - r.j0) == 1 ? 1 : 4;
+  r.kfast = point_order();
   const bool t = timing(name);
   if (t) time_begin(st);
   hipLaunchKernelGGL(kern, grid_of(r, by), dim3(kBx, by, 1), 0, st, r, 1, args...);
@@ -405,7 +407,7 @@ struct Piece {
   bool on;
 };
 __device__ __forceinline__ Piece level_piece(const Range& r, int lv) {
-  const Blk b = point_block(1);
+  const Blk b = point_block(r.kfast);
   Piece p;
   p.i = r.i0 + b.x * kBx + int(threadIdx.x);
   p.j = r.j0 + b.y * int(blockDim.y) + __builtin_amdgcn_readfirstlane(int(threadIdx.y));
@@ -4257,7 +4259,7 @@ struct ScPiece {
   bool on;
 };
 __device__ __forceinline__ ScPiece sc_piece(const Range& r, int lv) {
-  const Blk b = point_block(1);
+  const Blk b = point_block(r.kfast);
   const int np = (r.k1 - r.k0 + lv - 1) / lv;
   ScPiece p;
   p.i = r.i0 + b.x * kBx + int(threadIdx.x);

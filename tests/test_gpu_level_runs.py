@@ -6,10 +6,14 @@ FP32-bulk: the change of every field over the two steps is within 5 % (relative 
 by 6e-8 of it about ten times in two steps; the fields change by 1e-5 of their size or more in them, so rounding makes
 up to 2 % of the change, while a flux missing or misplaced at the seams of runs of 2 to 6 levels makes tens of per
 cent."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
-from conftest import bitwise_equal, first_diff
+from conftest import ROOT, bitwise_equal, first_diff
 from cppwrf_amd import _abi as A
 from cppwrf_amd.boundary import drifting_boundary
 from cppwrf_amd.dyn import Case, Context, RK3
@@ -69,3 +73,29 @@ def test_runs_of_levels(ctx, name):
         e = rel_l2(change[1], change[0])
         print(f"[level runs] {name} {A.FIELD_NAMES[fid]}: {e:.2e}", flush=True)
         assert e <= 5e-2, A.FIELD_NAMES[fid]
+
+
+_STEP = """
+import sys
+import numpy as np
+from cppwrf_amd import _abi as A
+from cppwrf_amd.dyn import Case, Context, RK3
+ctx = Context(0)
+for p in (A.MI_FP64, A.MI_FP32_BULK):
+    case = Case.hills(198, 121, 20, dx=15000.0, dt=60.0, seed=8)
+    d = RK3(ctx, case.grid, case.params(precision=p, time_step_sound=4, damp_opt=3, n_moist=2, n_scalars=2), case)
+    d.step(2)
+    np.save(f"{sys.argv[1]}_{p}.npy", np.concatenate([d.field(f).ravel() for f in case.STATE + (A.MI_Q, A.MI_Q + 1)]))
+"""
+
+
+def test_block_order_keeps_the_bits(ctx, tmp_path):
+    """MI_BLOCK_ORDER=ijk (read once per process) gives every point kernel's blocks, runs of levels included, the i, j,
+    level order: the same results"""
+    for order in ("", "ijk"):
+        print(f"[level runs] block order {order!r}", flush=True)
+        subprocess.run([sys.executable, "-c", _STEP, str(tmp_path / ("o" + order))], check=True, cwd=ROOT, timeout=100,
+                       env=dict(os.environ, MI_BLOCK_ORDER=order))
+    for p in (A.MI_FP64, A.MI_FP32_BULK):
+        a, b = (np.load(tmp_path / f"o{o}_{p}.npy") for o in ("", "ijk"))
+        assert bitwise_equal(a, b), p
