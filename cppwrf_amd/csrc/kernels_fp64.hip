@@ -205,14 +205,6 @@ void launch_level(const char* name, K kern, Range r, hipStream_t st, T... args) 
   hipLaunchKernelGGL(kern, grid_of(r, by), dim3(kBx, by, 1), 0, st, r, 1, args...);
   if (t) time_end(st, point_bytes(name) * double(r.i1 - r.i0) * double(r.j1 - r.j0) * double(r.k1 - r.k0));
 }
-template <class K, class... T>
-void launch_cols(const char* name, K kern, int nx, int ny, int nz, hipStream_t st, T... args) {
-  const bool t = timing(name);
-  if (t) time_begin(st);
-  hipLaunchKernelGGL(kern, dim3(unsigned((nx + kBx - 1) / kBx), unsigned(ny), 1), dim3(kBx, 1, 1), 0, st, args...);
-  if (t) time_end(st, point_bytes(name) * double(nx) * double(ny) * double(nz));
-}
-
 // ----------------------------------------------------------------------------- halo fill
 // One halo slot of one direction (reference semantics src/core/halo.cpp:52-84): slot a = 0..7 maps to
 // i = 0, -1, -2, -3, n, n+1, n+2, n+3 on face-staggered points and -1, -2, -3, n, n+1, n+2 otherwise.
@@ -2110,7 +2102,7 @@ __device__ __forceinline__ bool ring_blocks(const Args& a, const Blk& b, double*
 // within FP32-bulk's error bar.  FP64 keeps the reference's serial order (bit-identical).
 constexpr bool kScanChains = sizeof(real) == 4;
 // inclusive prefix sum over the lanes of a wavefront
-__device__ __forceinline__ double wave_prefix_sum(double v, int lane) {
+[[maybe_unused]] __device__ __forceinline__ double wave_prefix_sum(double v, int lane) {
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     const double t = __shfl_up(v, d, 64);
@@ -2564,7 +2556,7 @@ __device__ __forceinline__ void acoustic_levels(const Args& a, int bx, int j, do
   double* X1 = X0 + KT * CI;
   double* X2 = X1 + KT * CI;
   double* X3 = X2 + KT * CI;
-  double* Y0 = X3 + KT * CI;
+  double* Y0 = X3 + KT * CI;                      // four arrays per level and column, then one value per column
   const int L = (nz + 1) * CI;
   for (int e = int(threadIdx.x); e <= KT * LPT; e += int(blockDim.x)) {
     const int k = e > nz ? nz : e;
@@ -2772,11 +2764,10 @@ __device__ __forceinline__ void acoustic_levels(const Args& a, int bx, int j, do
   for (int q = 1; q < LPT; ++q) R[q] = rhs(q, wdn[q], wdn[q - 1]);
   // the neighbouring chunks' edge values: wdwn of the top and bottom layers, t_2ave and phi'' of the top level
   static_assert(LPT >= 2, "the chunk's top phi'' must not depend on the chunk below");
-  double* XB = Y0 + 4 * L + CI;
   X0[kt * CI + ci] = wdn[LPT - 1];
   X1[kt * CI + ci] = t2a[LPT - 1];
   X2[kt * CI + ci] = R[LPT - 1];
-  XB[kt * CI + ci] = wdn[0];
+  X3[kt * CI + ci] = wdn[0];
   __syncthreads();
   const bool below = kt > 0, above = kt + 1 < KT;
   const double wd_m = below ? X0[(kt - 1) * CI + ci] : 0.0;
@@ -2790,7 +2781,7 @@ __device__ __forceinline__ void acoustic_levels(const Args& a, int bx, int j, do
     dwt[q] = dampmag != 0.0 ? ld(f.dampwt + row, eo[q]) : real(0);
     wsv[q] = dampmag != 0.0 ? ld(f.w_save + row, eo[q]) : real(0);
   }
-  R[LPT] = rhs(LPT, above ? XB[(kt + 1) * CI + ci] : 0.0, wdn[LPT - 1]);
+  R[LPT] = rhs(LPT, above ? X3[(kt + 1) * CI + ci] : 0.0, wdn[LPT - 1]);
   // ---------------------------------------------------------------- 6: explicit w''
   double wk[LPT + 1];
   {
@@ -4905,11 +4896,12 @@ void launch_uv(const Args& a, double dts, hipStream_t st) {
 // LDS of k_acoustic_levels for blocks of ci columns x kt threads of lpt levels (the layout of acoustic_levels)
 size_t levels_lds_bytes(int ci, int kt, int lpt, int nz) {
   const size_t whole = size_t(4) * (nz + 1) * ci + ci;
-  return (size_t(kt * lpt + 1) * kAcCoef + size_t(5) * kt * ci + whole) * sizeof(double);
+  return (size_t(kt * lpt + 1) * kAcCoef + size_t(4) * kt * ci + whole) * sizeof(double);
 }
 bool levels_fit(int ci, int nz) {
   const int kt = (nz + kAcLpt) / kAcLpt;
-  return ci * kt <= 512 && levels_lds_bytes(ci, kt, kAcLpt, nz) <= kLdsMax;
+  // 8 columns up to 127 levels, 4 up to 225 (64 KB less one more array per chunk), then 2
+  return ci * kt <= 512 && levels_lds_bytes(ci, kt, kAcLpt, nz) + size_t(kt) * ci * sizeof(double) <= kLdsMax;
 }
 // the batched substep shapes: uv blocks of 64 x 4 points, acoustic blocks of 8 columns x 64 levels
 constexpr int kBatchCI = 8, kBatchKT = 64;
