@@ -31,12 +31,24 @@ def _hills(bc, seed, nz=20):
     return lambda: Case.hills(198, 121, nz, dx=15000.0, dt=60.0, seed=seed, bc=bc)
 
 
+def _bubble(nx, ny, nz, bc, **kw):
+    return lambda: Case.bubble3d(nx, ny, nz, seed=nz, noise_amp=0.3, bc=bc, bubble_zc=3000.0, **kw)
+
+
 CASES = {  # name: (case, parameters, the plugin's forcings kept)
     # the vapour stores RQVFTEN, level by level, beside species whose runs march: plain and limited, in one list or two
     "forcing_periodic": (_hills(P, 3), dict(n_moist=2, n_scalars=4, moist_adv_opt=1, scalar_adv_opt=0), True),
     "forcing_specified": (_hills(B, 4), dict(n_moist=3, n_scalars=3, moist_adv_opt=1), True),
     "forcing_plain": (_hills(P, 5), dict(n_moist=1, n_scalars=1, moist_adv_opt=0), True),
     "forcing_tracer_limited": (_hills(P, 6), dict(n_moist=1, n_scalars=2, moist_adv_opt=0, scalar_adv_opt=1), True),
+    # open sides: advance_uv, small_step_prep, calc_cq and the limiter's scale take runs there too
+    "open_limited": (_hills(O, 9), dict(n_moist=3, n_scalars=4, moist_adv_opt=1, scalar_adv_opt=1), False),
+    "open_dry": (_bubble(257, 190, 33, O, dx=3000.0, ztop=16000.0, dt=10.0), {}, False),
+    # the rigid lid, and updraughts beyond a vertical Courant number of 1 (set below) that w_damping pulls back
+    "lid_w_damping": (_bubble(198, 149, 24, P, dx=10000.0, ztop=8000.0, dt=20.0),
+                      dict(time_step_sound=8, top_lid=1, w_damping=1, zdamp=2000.0), False),
+    "specified_six": (_hills(B, 10, 23), dict(n_moist=6, n_scalars=6, moist_adv_opt=1, diff_6th_opt=1), False),
+    "lid_tall": (_bubble(130, 129, 70, P, dx=1000.0, ztop=18000.0, dt=2.0), dict(top_lid=1), False),
 }
 
 
@@ -60,11 +72,16 @@ def test_runs_of_levels(ctx, name):
             d.load_boundary(drifting_boundary(case, seed=5))
         for fid, q in (moist_species(case, ns, seed=7) if ns else {}).items():
             d.set_field(fid, q)
+        if kw.get("w_damping"):
+            z, _, x = np.indices(A.field_shape(A.MI_U, case.grid.nx, case.grid.ny, case.grid.nz))
+            d.set_field(A.MI_U, 180.0 * np.sin(2 * np.pi * x / 11) * (z < case.grid.nz // 2))
         if forcing:
             d.set_column_physics(Plugin(True, True, ns))
     before = [{f: d.field(f) for f in fids} for d in doms]
     for d in doms + [orc]:
-        d.step(2)
+        d.step(1)
+        assert not kw.get("w_damping") or d.cfl_max()[0] > 1.0
+        d.step(1)
     for fid in fids + ((A.MI_TH_FORCING, A.MI_QV_FORCING) if forcing else ()):
         a, b = doms[0].field(fid), orc.field(fid)
         assert bitwise_equal(a, b), f"{A.FIELD_NAMES[fid]}: {first_diff(a, b)}"
