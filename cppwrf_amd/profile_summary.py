@@ -36,6 +36,8 @@ def kernel_key(name: str):
     short = m.group(1) if m else name.split("(")[0][-40:]
     t = re.search(r"k_[a-z0-9_]+<([^>]*)>", name)
     shape = t.group(1).replace(", ", "x").replace(",", "x") if t else "-"
+    if short == "acoustic_levels":  # one of the substep kernel's shapes: columns per block, levels per thread, scans
+        short, shape = "acoustic", "levels:" + shape
     return short, mode, shape
 
 
