@@ -277,7 +277,7 @@ struct Domain final : mi_domain {
   // No kernel between the stage's prologue and its end reads a halo point: the substep kernels reach their neighbour
   // columns through the lateral boundary condition (a periodic side's column n is column 0, a mirrored or copied one
   // its inner column).  So the reference's refreshes after the prologue, after advance_uv and after advance_mu_t and
-  // advance_w (small_step.cpp:517-522, 540-541, 572, 593) are left out: 21 launches of a dry step with 6 acoustic steps.
+  // advance_w (small_step.cpp:517-522, 540-541, 572, 593) are left out: 23 launches of a dry step with 6 acoustic steps.
   // The stage's last refreshes write every halo a later kernel reads.
   int stage_ns(int rk) const { return rk == 1 ? 1 : (rk == 2 ? n_sound_ / 2 : n_sound_); }
   double stage_dts(int rk) const { return rk == 1 ? grid.dt / 3.0 : grid.dt / n_sound_; }

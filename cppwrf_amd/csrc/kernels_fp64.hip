@@ -609,6 +609,11 @@ __device__ __forceinline__ double open_y_scalar(const Geo& g, const T* q, const 
 // the per-level kernels' below, operand for operand; the marches take the rows whose y fluxes have the domain's own
 // order and the wavefronts without an open edge, the per-level code the others.  Columns next to a specified or open x
 // side pick their x flux's order lane by lane.
+//
+// Bound by latency, at the wavefronts their registers leave: u, v 134, 138 VGPRs and 16 B of scratch, 3 wavefronts per SIMD
+// in FP32-bulk (198, 206 and 2 in FP64); w 115 and 4 (157 and 3); theta 56 and 8 (95 and 5); phi 109 and 4 (126 and 4).
+// Per launch at 425x300x50 against one level per thread (kernel traces): u 246 -> 216, v 229 -> 203, w 178 -> 155, phi 141 ->
+// 128 us, theta even at 94 in FP32-bulk; FP64 u 316 -> 308, v 367 -> 321, phi 218 -> 193, w and theta 1-2 % longer, 253 and 161.
 // KTendU (DIR 0) and KTendV (DIR 1): the same terms with the two directions exchanged
 template <int DIR>
 __device__ __forceinline__ void tend_uv_levels(const Args& a, int i, int j, int ka, int kb) {
@@ -1825,7 +1830,7 @@ MI_COLUMN_KERNEL k_ss_column(Args a, double cof, double dts) {
 // n - 1): no halo point is read.  All of a level's loads are unconditional and issued together.  Measured against one
 // level per thread (78 loads per point and level, 460 scalar instructions of prologue; latency-bound at 31 % vector
 // issue): 425x300x50 FP32-bulk 177 -> 118 us per launch, FP64 283 -> 206.  It is bounded by the loads in flight per
-// wavefront (113 VGPRs in FP32-bulk, four wavefronts per SIMD).
+// wavefront (117 VGPRs in FP32-bulk, four wavefronts per SIMD; 162 and three in FP64).
 //
 // FP32-bulk: the same update with the bulk arithmetic in FP32 (one multiply by a rounded reciprocal per division); the
 // differences of the full geopotential php and of the base pressure pb are taken in FP64 first.
@@ -2506,10 +2511,12 @@ MI_COLUMN_KERNEL k_acoustic(Args a, double dts, int it, int ns) {
 // FP32-bulk with two levels per thread takes 161 VGPRs, three wavefronts per SIMD; bounded to four it spills and runs
 // slower (628 us at 425x300x50 with blocks of 16 columns), as four levels per thread (717 us) do.  Blocks of 8 columns
 // (four wavefronts, three blocks per CU) beat 16 and 4 columns.  Substep kernel, FP32-bulk, per launch, against the
-// level-per-thread blocks of 8 x 64: 425x300x50 557 -> 446 us (475 with
-// the spec zone's columns, 29 us in a launch of their own); the step of 219x173x44 3.24 -> 2.65 ms with
-// advance_uv below and without the substeps' halo launches.  In FP64 (197 VGPRs, two wavefronts per SIMD) it is
-// slower (704 -> 775 us), so FP64 keeps the level-per-thread form by default.
+// level-per-thread blocks of 8 x 64: 425x300x50 557 -> 446 us (459 to 478 over three cards with the spec zone's columns, 29 us
+// in a launch of their own); the step of 219x173x44 3.24 -> 2.65 ms with advance_uv below and without the substeps' halo
+// launches.  It reads the level above each pair again, as the chunk above does: 1186 MB moved per launch at 425x300x50, 1.19
+// times its arrays (the level-per-thread form 1.12 times).  In FP64 (197 VGPRs, two wavefronts per SIMD) the forms are close:
+// a step of 425x300x50 21.33 ms level per thread, 21.48 so, 119x89x44 1.928 and 1.982 ms (the spec zone a launch of its own),
+// dry 219x173x44 4.21 and 4.12 ms.  FP64 keeps the level-per-thread form by default; the autotuner tries both.
 //
 // A level k of a column beyond nz (the last chunk) and an idle lane read clamped addresses and store nothing.
 constexpr int kAcCoef = 10;  // doubles per level of the LDS coefficient table
@@ -4832,7 +4839,8 @@ bool col_cfg_fits(int kernel, int cfg, int nz) {
 int col_cfg_default(int kernel, int nx, int ny, int nz) {
   // the substep kernel: the narrowest one-level-per-thread shape; the others by the number of columns
   if (kernel == kColAcoustic) {
-    // FP32-bulk: several levels per thread (425x300x50 557 -> 446 us; FP64 is slower that way, 704 -> 775 us)
+    // FP32-bulk: several levels per thread (425x300x50 557 -> 446 us).  FP64: level per thread, 1-3 % faster with a spec
+    // zone, 2 % slower on a dry 219x173x44 (acoustic_levels)
     if (kAcFp32) return kColLevels;
     for (int c : {4, 5, 6})
       if (col_cfg_fits(kernel, c, nz)) return c;
