@@ -1,7 +1,6 @@
-// The library's choice of the column kernels' block shapes by the number of columns, and of the substep kernel's form, for
-// a domain alone and for a batch, on grids whose row block is below, at and above 2^29 elements: the form with several
-// levels per thread reaches it with 32-bit byte offsets.  Built for each arithmetic (MI_REAL, MI_NS) and linked with the
-// library; nothing is launched.
+// The library's choice of the substep kernel's form, for a domain alone and for a batch, on grids whose row block is
+// below, at and above 2^29 elements: the form with several levels per thread reaches it with 32-bit byte offsets.  Built
+// for each arithmetic (MI_REAL, MI_NS) and linked with the library; nothing is launched.
 #include <cstdio>
 
 #include "../../cppwrf_amd/csrc/kernels_fp64.hpp"
@@ -42,15 +41,6 @@ int main() {
   const Args* mixed[] = {&small, &below, &at};
   expect("two small members", batch_levels(mixed, 2), f32);
   expect("a large member among small ones", batch_levels(mixed, 3), 0);
-  // the stage's column kernels by the number of columns: 64 columns x 4 threads only where they were the faster blocks
-  const int few = 4, mid = 0, many = 7;
-  const struct { int nx, ny, want; } grids[] = {{24, 24, few}, {56, 56, few}, {64, 64, mid}, {119, 89, mid}, {129, 129, mid},
-                                                {140, 140, mid}, {150, 150, mid}, {160, 160, many}, {219, 173, many}, {425, 300, many}};
-  for (const auto& g : grids)
-    for (int kernel : {kColLargePrep, kColFinish}) {
-      expect("the default shape", col_cfg_default(kernel, g.nx, g.ny, 44), g.want);
-      expect("the stage's column kernel", col_cfg_default(kColSsColumn, g.nx, g.ny, 44), g.want == many ? mid : g.want);
-    }
   std::printf("%d wrong\n", bad);
   return bad ? 1 : 0;
 }
