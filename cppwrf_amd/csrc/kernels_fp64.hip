@@ -4851,7 +4851,13 @@ int col_cfg_default(int kernel, int nx, int ny, int nz) {
   // waste less of a cache line (large_prep, ss_column, finish FP32-bulk: 64x64x40 20.8, 15.4, 14.8 -> 18.0, 16.9, 14.2 us;
   // 119x89x44 33.1, 32.5, 24.4 -> 23.9, 23.1, 20.9 us).  On large grids 64 columns x 4, a wavefront a row, where the work
   // is the loads and stores (large_prep, finish: 425x300x50 187, 232 -> 138, 187 us, but 119x89x44 23.9, 20.9 -> 27.6,
-  // 34.9 us: too few blocks); the ss column's three LDS arrays do not fit that shape.
+  // 34.9 us: too few blocks); the ss column's three LDS arrays do not fit that shape.  Both sides of the two lines, dry
+  // steps with 6 acoustic steps of a domain alone, FP32-bulk / FP64: 56x56x40 505 / 621 us with the shapes of few columns,
+  // 516 / 635 with 16 x 16, 64x64x40 550 / 669 and 542 / 668, 80x80x40 800 / 1059 and 769 / 1027; 110x110x44 1003 / 1523 us
+  // with 16 x 16, 1033 / 1549 with 64 x 4, 129x129x44 1275 / 2197 and 1304 / 2221, 150x150x44 1502 / 2735 and 1509 / 2735,
+  // 160x160x44 1694 / 3117 and 1692 / 3097, 180x180x44 2109 / 3779 and 2083 / 3751.  So alone the second line would lie at
+  // 24000 columns; members of a batch fill the chip together, and there 64 x 4 wins from less (8 members of 5500 to 26500
+  // columns: 8.57 / 14.37 ms a step with the line at 16384, 8.63 / 14.44 with it at 24576).
   const int64_t cols = int64_t(nx) * ny;
   const bool small = cols < 4096, large = cols > 16384;
   const int pref[] = {small ? (nz + 1 <= 64 ? 4 : (nz + 1 <= 128 ? 5 : 6)) : (large && kernel != kColSsColumn ? 7 : 0), 0, 3, 5, 6};
