@@ -1,8 +1,8 @@
 """The HBM traffic that bench.py reports for a kernel is the one of the shape the workload launched most, the form of the
 substep kernel with several levels per thread among its shapes."""
 import csv
+import os
 
-import bench
 from cppwrf_amd import profile_summary as PS
 from cppwrf_amd.serving import alloc_elems
 
@@ -19,6 +19,8 @@ def _counters(d, counter, rows):
 
 
 def test_traffic_of_the_launched_substep_form(tmp_path, monkeypatch):
+    monkeypatch.setattr(os, "environ", dict(os.environ))  # bench sets OpenMP's thread binding for its own process
+    import bench
     n3 = alloc_elems(20, 16, 12)
     copy = (5 * 4 * n3 + 8 * (n3 // 13)) / 1024.0  # KiB, so both scale factors are 1
     rows = [("k_copy_step", copy, 3), ("k_acoustic<8, 64>", 1000.0, 4), ("k_acoustic_levels<8, 2, true>", 700.0, 30),
